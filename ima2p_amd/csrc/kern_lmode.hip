@@ -7,16 +7,16 @@
 // layout (ginfo.cpp:288-316): cc | fc | hcc (npsize each), mc | fm (nmig
 // each), qintegrate (npsize), mintegrate (nmig), pdg, probg, split times.
 //
-// Mapping (jointp): one workgroup of 256 lanes per (tile of points, chunk
-// of rows), each lane carrying one or two points.  The workgroup stages
-// its rows in LDS as compact FP64 records that no longer depend on the
-// point, and every lane walks them in order, so each row is read from HBM
-// once per point tile and broadcast from LDS; a point's coefficients sit
-// in registers.  Chunk partials are merged by a second kernel in chunk
-// order.  The chunk size depends on the table only, never on how many
-// points share a launch, so a point's result is the same alone and batched
-// with others.  margincalc: one thread per value, 64-value tiles.
+// jointp is a matrix product on the FP64 matrix unit, genealogies times
+// points, with an exp and a sum over the genealogies behind it (see below).
+// Chunk partials are merged by a second kernel in a fixed order, and the
+// rows a lane works on depend on the table only, never on how many points
+// share a launch, so a point's result is the same alone and batched with
+// others.  margincalc: one thread per value, 64-value tiles.
 #include <float.h>
+#include <limits.h>
+
+#include <algorithm>
 
 #include "ima_internal.h"
 #include "prior_math.h"
@@ -44,60 +44,118 @@ __host__ __device__ inline JointLayout joint_layout(int npsize, int nmig) {
   return L;
 }
 
-// eexp (utilities.cpp:1507-1539): e^x as m * 10^z, with a degree-10 Taylor
-// series of e^u on u = x - n ln2 in [0, ln2).  Coefficients are 1/k!.
-__device__ inline void d_eexp(double x, double *m, int *z) {
-  const double LOG_10_2 = 0.30102999566398119521;
-  const int nn = (int)floor(x / kLn2);
-  double zr = LOG_10_2 * (double)nn;
-  *z = (int)zr;
-  zr -= (double)*z;
-  const double u = x - (((double)nn) * kLn2);
-  const double temp = 1 + u * (1.0 + u * (0.5 + u * (0.16666666666666666666666666667 +
-      u * (0.04166666666666666666666666667 + u * (0.00833333333333333333333333333 +
-      u * (0.001388888888888888888888888889 + u * (0.000198412698412698412698412698 +
-      u * (0.000024801587301587301587301587301 + u * (2.75573192239858906525573192239859e-6 +
-      u * (2.75573192239858906525573192239e-7))))))))));
-  *m = temp * pow(10.0, zr);
-  if (fabs(*m) > 10) {
-    *m = *m / 10.0;
-    *z = *z + 1;
-  }
-  if (fabs(*m) < 1) {
-    *m = *m * 10.0;
-    *z = *z - 1;
-  }
-}
-
 struct LArgs {
   const float *rows;
   int G, K, npsize, nmig, npops, modeltype, r0, r1;
   const double *x;  // [npoints][np]
-  int npoints, nchunks, chunk_rows, stage;
+  int npoints, nchunks, chunk_rows;
 };
 
-// --------------------------------------------------------------- EXACT --
-// Per (point, chunk): running max M and s = sum exp(p - M), s2 = sum
-// exp(2(p - M)) for the effective sample number.
-// Staging folds each row into a compact FP64
-// record that no longer depends on the point: c0 = (the row's base term)
-// minus the hcc of the parameters in range, then (count, weight) of each
-// parameter in [r0, r1).  A point's term is then
-//   p = c0 + sum_k count_k * A_k + weight_k * F_k
-// with A = log 2 - log x (theta, models 0/1; else 0) or log x (migration),
-// F = -2/x (theta: 2 fc / x) or -x (migration); (2/x) fc equals (2 fc)/x
-// exactly, the remaining differences from the reference's order are the
-// fused multiply-adds and the summation order (about 1e-16 relative).
-// 256 lanes per workgroup share one staged block; each lane carries PTS
-// points, so every record read from LDS serves PTS independent exp chains.
 constexpr int kXLanes = 256;
 
-__host__ __device__ inline int xrec_len(int nr) { return 1 + 2 * nr; }
 
-__device__ inline void stage_compact(const LArgs &a, double *sh, int g0, int cnt, int nr) {
+// ------------------------------------------------------------- jointp --
+// A point's term for a genealogy is
+//   p = c0 + sum_k count_k * A_k + weight_k * F_k
+// with c0 = (the row's base term) minus the hcc of the parameters in range,
+// A = log 2 - log x (theta, models 0/1; else 0) or log x (migration), F =
+// -2/x (theta: 2 fc / x) or -x (migration); (2/x) fc equals (2 fc)/x
+// exactly, the remaining differences from the reference's order are the
+// fused multiply-adds and the summation order (about 1e-16 relative).  A
+// batch of points against a table is therefore a matrix product, genealogies
+// x (1 + 2 parameters) x points, followed by an exp and a sum over the
+// genealogies.  It runs on the FP64 matrix unit, in logarithms to base 2
+// (the points' coefficients carry log2 e), so a term is 2^(p - M) without a
+// split-constant reduction.
+//
+// One workgroup of four wavefronts takes one chunk of rows and up to
+// 16 * T points.  It stages kRows rows at a time in LDS as FP64 records
+// [c0, count_0, weight_0, ...]; each wavefront multiplies its quarter of
+// them, 16 rows a tile, with every tile of 16 points.  A lane of the product
+// holds one point and four consecutive rows of a tile; it keeps that point's
+// running maximum and sums over its own rows, so no lane talks to another
+// until the end of the chunk, where the 16 partials of a point (4 wavefronts
+// x 4 lanes) are merged in a fixed order.  The rows a lane sees depend on
+// the table and the parameter range alone: a point's value is the same
+// alone and batched with others.
+//
+// Bound: FP64 issue, 18 vector operations per (point, genealogy) pair
+// (subtract, round, 11 multiply-adds, ldexp, the maximum and two sums; 2.2 ns
+// per 64 lanes) and the product (48 ns per 16 x 16 x 4 on a SIMD).  The two
+// share their issue here: a loop of half of each takes the sum of both.
+// Multiply-adds in place of the product would cost 22 ns instead of 36 per
+// 64 pairs at five parameters, but the row values then pass through LDS once
+// per lane: 4.5 ms where this takes 3.9 (4096 points on 1e6 genealogies).
+// With one lane per point (rows in order, the library's exp and a branch on
+// every new maximum) that surface took 6.45 ms, 500 points on 1e5 in
+// REF_COMPAT 277 us, and one point on 1e5 171 us (one lane of 256 working);
+// here 4.0 ms, 111 us and 13 us.
+typedef double dvec4 __attribute__((ext_vector_type(4)));
+
+constexpr double kLog2E = 1.4426950408889634074;
+constexpr double kBadCoef = 1e250;  // |count or weight| <= 3.4e38: no overflow below it
+constexpr double kPadRow = -1e300;  // c0 of the rows past the end: 2^(p - M) = 0
+
+template <int NR>
+struct XShape {
+  static constexpr int kRows = NR <= 8 ? 256 : 128;    // staged at a time
+  static constexpr int kRT = kRows / 64;               // row tiles per wavefront
+  // matrix steps of 4: the parameters' counts and weights, and c0 as one
+  // more operand where they leave room, else as the product's addend
+  static constexpr bool kAdd = (2 * NR) % 4 == 0;
+  static constexpr int kSteps = (2 * NR + 3) / 4;
+  static constexpr int kKP = 4 * kSteps;  // record length, zero padded
+  // distance of records: 24, 40, 56 or (padded) 4 mod 8 dwords, so that the
+  // rows of a fragment load spread over the banks
+  static constexpr int kStride = kKP + (kKP % 8 == 0 ? 2 : 0);
+  static constexpr int kLds = kRows * kStride + (kAdd ? kRows : 0);
+  // place of parameter k's count in a record (its weight follows)
+  static __device__ __forceinline__ constexpr int at(int k) { return (kAdd ? 0 : 1) + 2 * k; }
+  static constexpr int kEnd = (kAdd ? 0 : 1) + 2 * NR;
+};
+
+// 2^(f + n), f in [-1/2, 1/2], exactly 2^n at f = 0: a polynomial of degree
+// 11 (interpolation at the Chebyshev nodes, 2e-17 relative), scaled.
+__device__ __forceinline__ double exp2_scaled(double f, int n) {
+  double p = 4.4558179083360645e-10;
+  p = fma(p, f, 7.074194297288521e-09);
+  p = fma(p, f, 1.0178057087733941e-07);
+  p = fma(p, f, 1.3215432535912375e-06);
+  p = fma(p, f, 1.5252733841556773e-05);
+  p = fma(p, f, 0.00015403530463724353);
+  p = fma(p, f, 0.001333355814640647);
+  p = fma(p, f, 0.009618129107587256);
+  p = fma(p, f, 0.055504108664821625);
+  p = fma(p, f, 0.24022650695910158);
+  p = fma(p, f, 0.6931471805599453);
+  p = fma(p, f, 1.0);
+  return ldexp(p, n);
+}
+// 2^t; the conversion to int saturates, so any finite t below the range
+// gives 0
+__device__ __forceinline__ double exp2_fast(double t) {
+  const double n = rint(t);
+  return exp2_scaled(t - n, (int)n);
+}
+// 2^t for any t <= 0, infinite or NaN too
+__device__ __forceinline__ double exp2_any(double t) { return t < -1100.0 ? 0.0 : exp2_fast(t); }
+
+// Rows [g0, g0 + cnt) as records in sh, rows cnt .. kRows - 1 as padding.
+// Returns whether this thread met a value that is not finite.
+template <int NR>
+__device__ inline bool stage_rows(const LArgs &a, double *sh, int g0, int cnt) {
+  using X = XShape<NR>;
   const JointLayout L = joint_layout(a.npsize, a.nmig);
-  const int rl = xrec_len(nr);
-  for (int r = threadIdx.x; r < cnt; r += blockDim.x) {
+  bool bad = false;
+  for (int r = threadIdx.x; r < X::kRows; r += kXLanes) {
+    double *o = sh + r * X::kStride;
+    double *c0 = X::kAdd ? sh + X::kRows * X::kStride + r : o;
+    if (r >= cnt) {
+#pragma unroll
+      for (int k = 0; k < X::kKP; ++k) o[k] = 0.0;
+      *c0 = kPadRow;
+      continue;
+    }
     const float *g = a.rows + (size_t)(g0 + r) * a.K;
     double base;
     if (a.npops == 2) {
@@ -110,148 +168,280 @@ __device__ inline void stage_compact(const LArgs &a, double *sh, int g0, int cnt
         for (int i = 0; i < a.nmig; ++i) t += (double)g[L.mip + i];
       base = -t;
     }
-    double *o = sh + (size_t)r * rl;
-    for (int k = 0; k < nr; ++k) {
-      const int i = a.r0 + k;
-      if (i < a.npsize) {
-        base -= (double)g[L.hccp + i];
-        o[1 + 2 * k] = (double)g[L.ccp + i];
-        o[2 + 2 * k] = (double)g[L.fcp + i];
-      } else {
-        o[1 + 2 * k] = (double)g[L.mcp + i - a.npsize];
-        o[2 + 2 * k] = (double)g[L.fmp + i - a.npsize];
-      }
-    }
-    o[0] = base;
-  }
-}
-
-// Per-point coefficients of the compact records: A = log 2 - log x
-// (theta, models 0/1; else 0) or log x (migration), F = -2/x or -x.
-template <int NR>
-__device__ inline void point_coef_compact(const LArgs &a, const double *xp, double (&A)[NR],
-                                          double (&F)[NR]) {
-#pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const int i = a.r0 + k;
-    const double x = xp[i];
-    if (i < a.npsize) {
-      A[k] = (a.modeltype == 0 || a.modeltype == 1) ? kLn2 - log(x) : 0.0;
-      F[k] = -2.0 * (1.0 / x);
-    } else {
-      A[k] = log(x);
-      F[k] = -x;
-    }
-  }
-}
-
-template <int NR>
-__device__ inline double compact_term(const double *v, const double (&A)[NR],
-                                      const double (&F)[NR]) {
-  double p = v[0];
-#pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    p = fma(v[1 + 2 * k], A[k], p);
-    p = fma(v[2 + 2 * k], F[k], p);
-  }
-  return p;
-}
-
-template <int NR, int PTS>
-__global__ __launch_bounds__(kXLanes) void jointp_exact_fast(LArgs a, double *work) {
-  extern __shared__ double shrows[];
-  const int np = a.npsize + a.nmig;
-  double A[PTS][NR], F[PTS][NR], M[PTS], s[PTS], s2[PTS];
-  int pt[PTS];
-#pragma unroll
-  for (int j = 0; j < PTS; ++j) {
-    pt[j] = blockIdx.x * (kXLanes * PTS) + j * kXLanes + threadIdx.x;
-    const double *xp = a.x + (size_t)(pt[j] < a.npoints ? pt[j] : 0) * np;
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
       const int i = a.r0 + k;
-      const double x = xp[i];
+      double c, w;
       if (i < a.npsize) {
-        A[j][k] = (a.modeltype == 0 || a.modeltype == 1) ? kLn2 - log(x) : 0.0;
-        F[j][k] = -2.0 * (1.0 / x);
+        base -= (double)g[L.hccp + i];
+        c = (double)g[L.ccp + i];
+        w = (double)g[L.fcp + i];
       } else {
-        A[j][k] = log(x);
-        F[j][k] = -x;
+        c = (double)g[L.mcp + i - a.npsize];
+        w = (double)g[L.fmp + i - a.npsize];
       }
+      o[X::at(k)] = c;
+      o[X::at(k) + 1] = w;
+      bad = bad || !isfinite(c) || !isfinite(w);
     }
-    M[j] = -DBL_MAX;
-    s[j] = 0.0;
-    s2[j] = 0.0;
+    bad = bad || !isfinite(base);
+#pragma unroll
+    for (int k = X::kEnd; k < X::kKP; ++k) o[k] = 0.0;
+    *c0 = base * kLog2E;
   }
-  const int chunk = blockIdx.y;
-  const int gbeg = chunk * a.chunk_rows;
-  const int gend = min(a.G, gbeg + a.chunk_rows);
-  constexpr int RL = 1 + 2 * NR;
-  for (int g0 = gbeg; g0 < gend; g0 += a.stage) {
-    const int cnt = min(a.stage, gend - g0);
-    __syncthreads();
-    stage_compact(a, shrows, g0, cnt, NR);
-    __syncthreads();
-    for (int r = 0; r < cnt; ++r) {
-      const double *o = shrows + (size_t)r * RL;
-      double v[RL];
-#pragma unroll
-      for (int q = 0; q < RL; ++q) v[q] = o[q];
-#pragma unroll
-      for (int j = 0; j < PTS; ++j) {
-        double p = v[0];
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-          p = fma(v[1 + 2 * k], A[j][k], p);
-          p = fma(v[2 + 2 * k], F[j][k], p);
-        }
-        if (p > M[j]) {
-          const double sc = exp(M[j] - p);
-          s[j] = s[j] * sc + 1.0;
-          s2[j] = s2[j] * sc * sc + 1.0;
-          M[j] = p;
-        } else {
-          const double w = exp(p - M[j]);
-          s[j] += w;
-          s2[j] = fma(w, w, s2[j]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < PTS; ++j)
-    if (pt[j] < a.npoints) {
-      double *o = work + ((size_t)pt[j] * a.nchunks + chunk) * 3;
-      o[0] = M[j];
-      o[1] = s[j];
-      o[2] = s2[j];
-    }
+  return bad;
 }
+
+// The points' coefficients, [tile][k][16], from point pt0 on (points past
+// the end repeat the last one); ptbad[tile * 16 + j] flags a point whose
+// terms might overflow.
+template <int NR, int T>
+__device__ inline void stage_points(const LArgs &a, double *sh, int *ptbad, int pt0) {
+  using X = XShape<NR>;
+  const int np = a.npsize + a.nmig;
+  for (int x = threadIdx.x; x < T * 16; x += kXLanes) ptbad[x] = 0;
+  __syncthreads();
+  for (int x = threadIdx.x; x < T * 16 * NR; x += kXLanes) {
+    const int p = x / NR, k = x % NR, i = a.r0 + k;
+    const double v = a.x[(size_t)min(pt0 + p, a.npoints - 1) * np + i];
+    double A, F;
+    if (i < a.npsize) {
+      A = (a.modeltype == 0 || a.modeltype == 1) ? kLn2 - log(v) : 0.0;
+      F = -2.0 * (1.0 / v);
+    } else {
+      A = log(v);
+      F = -v;
+    }
+    A *= kLog2E;
+    F *= kLog2E;
+    if (!(fabs(A) < kBadCoef) || !(fabs(F) < kBadCoef)) ptbad[p] = 1;
+    double *o = sh + ((size_t)(p / 16) * X::kKP) * 16 + p % 16;
+    o[X::at(k) * 16] = A;
+    o[(X::at(k) + 1) * 16] = F;
+  }
+  for (int p = threadIdx.x; p < T * 16; p += kXLanes) {
+    double *o = sh + ((size_t)(p / 16) * X::kKP) * 16 + p % 16;
+    if (!X::kAdd) o[0] = 1.0;
+    for (int k = X::kEnd; k < X::kKP; ++k) o[k * 16] = 0.0;
+  }
+  __syncthreads();
+}
+
+// Operand fragments.  The matrix unit gives lane l the rows l / 16 + 4 i of
+// the product (i = 0..3) and column l % 16; operand row i of a tile is
+// loaded from staged row 4 (i % 4) + i / 4, so the lane's four values are
+// the consecutive rows 4 (l / 16) .. + 3.
+template <int NR>
+struct RowFrag {
+  double v[XShape<NR>::kRT][XShape<NR>::kSteps];
+  dvec4 c0[XShape<NR>::kRT];  // the lane's rows' c0, or zero
+  __device__ __forceinline__ void load(const double *sh, int wave, int lane) {
+    using X = XShape<NR>;
+    const int i = lane & 15, row = 4 * (i & 3) + (i >> 2);
+#pragma unroll
+    for (int t = 0; t < X::kRT; ++t) {
+      const double *o = sh + (size_t)((wave * X::kRT + t) * 16 + row) * X::kStride + (lane >> 4);
+#pragma unroll
+      for (int s = 0; s < X::kSteps; ++s) v[t][s] = o[4 * s];
+      const double *c = sh + X::kRows * X::kStride + (wave * X::kRT + t) * 16 + 4 * (lane >> 4);
+      c0[t] = X::kAdd ? dvec4{c[0], c[1], c[2], c[3]} : dvec4{0.0, 0.0, 0.0, 0.0};
+    }
+  }
+};
 
 template <int NR>
-hipError_t launch_exact_fast(const LArgs &a, dim3 grid_y, size_t lds, hipStream_t st,
-                             double *work) {
-  constexpr int PTS = NR <= 8 ? 2 : 1;
-  const dim3 grid((a.npoints + kXLanes * PTS - 1) / (kXLanes * PTS), grid_y.y);
-  hipLaunchKernelGGL((jointp_exact_fast<NR, PTS>), grid, dim3(kXLanes), lds, st, a, work);
-  return hipSuccess;
+struct PointFrag {
+  double v[XShape<NR>::kSteps];
+  __device__ __forceinline__ void load(const double *sh, int tile, int lane) {
+    using X = XShape<NR>;
+    const double *o = sh + ((size_t)tile * X::kKP + (lane >> 4)) * 16 + (lane & 15);
+#pragma unroll
+    for (int s = 0; s < X::kSteps; ++s) v[s] = o[s * 64];
+  }
+};
+
+// log2 terms of the lane's point for rows 4 (lane / 16) + i of row tile t
+template <int NR>
+__device__ __forceinline__ void terms(const RowFrag<NR> &a, const PointFrag<NR> &b,
+                                      dvec4 (&p)[XShape<NR>::kRT]) {
+  using X = XShape<NR>;
+#pragma unroll
+  for (int t = 0; t < X::kRT; ++t) p[t] = a.c0[t];
+#pragma unroll
+  for (int s = 0; s < X::kSteps; ++s)
+#pragma unroll
+    for (int t = 0; t < X::kRT; ++t)
+      p[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.v[t][s], b.v[s], p[t], 0, 0, 0);
 }
 
-__global__ void jointp_exact_final(LArgs a, const double *work, double *out, double *ess) {
-  const int pt = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pt >= a.npoints) return;
-  const double *w = work + (size_t)pt * a.nchunks * 3;
-  double M = -DBL_MAX;
-  for (int c = 0; c < a.nchunks; ++c) M = fmax(M, w[c * 3]);
-  double s = 0.0, s2 = 0.0;
-  for (int c = 0; c < a.nchunks; ++c) {
-    if (w[c * 3 + 1] == 0.0) continue;
-    const double sc = exp(w[c * 3] - M);
-    s += w[c * 3 + 1] * sc;
-    s2 += w[c * 3 + 2] * sc * sc;
+// The largest, and the x-th, of a lane's values.
+template <int NR>
+__device__ __forceinline__ double largest(const dvec4 (&p)[XShape<NR>::kRT]) {
+  double m = fmax(fmax(p[0][0], p[0][1]), fmax(p[0][2], p[0][3]));
+#pragma unroll
+  for (int t = 1; t < XShape<NR>::kRT; ++t)
+    m = fmax(m, fmax(fmax(p[t][0], p[t][1]), fmax(p[t][2], p[t][3])));
+  return m;
+}
+template <int NR>
+__device__ __forceinline__ double pick(const dvec4 (&p)[XShape<NR>::kRT], int x) {
+  double v = p[0][0];
+#pragma unroll
+  for (int k = 1; k < 4 * XShape<NR>::kRT; ++k) v = x == k ? p[k / 4][k % 4] : v;
+  return v;
+}
+
+// Chunk and first point of this workgroup.
+struct XPlace {
+  int pt0, chunk, gbeg, gend, wave, lane;
+  int part;  // wavefront * 4 + lane group
+  int row0;  // the lane's first row of a stage (16 on per row tile)
+};
+template <int NR, int T>
+__device__ __forceinline__ XPlace x_place(const LArgs &a) {
+  XPlace w;
+  w.pt0 = blockIdx.x * (16 * T);
+  w.chunk = blockIdx.y;
+  w.gbeg = w.chunk * a.chunk_rows;
+  w.gend = min(a.G, w.gbeg + a.chunk_rows);
+  w.wave = threadIdx.x / kWave;
+  w.lane = threadIdx.x & (kWave - 1);
+  w.part = threadIdx.x / 16;
+  w.row0 = w.wave * XShape<NR>::kRT * 16 + 4 * (w.lane >> 4);
+  return w;
+}
+
+// --------------------------------------------------------------- EXACT --
+// Per (point, chunk): a reference M (base 2) and s = sum 2^(p - M), s2 = sum
+// 2^(2(p - M)) for the effective sample number.  M is a value the lane met
+// and at most 2^kSlack below its largest: FP64's range takes the difference,
+// so sums are rescaled when a term leaves it, not on every new maximum.
+struct XPart {
+  double M, s, s2;
+};
+constexpr double kSlack = 200.0;
+
+template <int NR, int T>
+__global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work) {
+  using X = XShape<NR>;
+  extern __shared__ double sh[];
+  double *shp = sh + X::kLds;
+  __shared__ int ptbad[T * 16];
+  const XPlace w = x_place<NR, T>(a);
+  stage_points<NR, T>(a, shp, ptbad, w.pt0);
+  PointFrag<NR> b[T];
+  double M[T], s[T], s2[T];
+  bool pbad[T];
+#pragma unroll
+  for (int j = 0; j < T; ++j) {
+    b[j].load(shp, j, w.lane);
+    pbad[j] = ptbad[j * 16 + (w.lane & 15)] != 0;
+    M[j] = -DBL_MAX;
+    s[j] = s2[j] = 0.0;
   }
-  out[pt] = log((double)a.G) - (M + log(s));
-  if (ess) ess[pt] = s * s / s2;
+  for (int g0 = w.gbeg; g0 < w.gend; g0 += X::kRows) {
+    const int cnt = min(X::kRows, w.gend - g0);
+    __syncthreads();
+    const bool rbad = __syncthreads_or(stage_rows<NR>(a, sh, g0, cnt)) != 0;
+    if (w.wave * (X::kRows / 4) >= cnt) continue;  // only padding in this quarter
+    RowFrag<NR> r;
+    r.load(sh, w.wave, w.lane);
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      dvec4 p[X::kRT];
+      terms<NR>(r, b[j], p);
+      if (rbad || pbad[j]) {
+        // infinities and NaN: one value after another, as they come
+#pragma unroll 1
+        for (int x = 0; x < 4 * X::kRT; ++x) {
+          if (w.row0 + x / 4 * 16 + x % 4 >= cnt) continue;
+          const double v = pick<NR>(p, x);
+          const bool up = v > M[j];
+          const double e = exp2_any(up ? M[j] - v : v - M[j]);
+          s[j] = up ? s[j] * e + 1.0 : s[j] + e;
+          s2[j] = up ? s2[j] * e * e + 1.0 : fma(e, e, s2[j]);
+          M[j] = up ? v : M[j];
+        }
+        continue;
+      }
+      const double m = largest<NR>(p);
+      if (__any(m - M[j] > kSlack)) {
+        // the reference moves up to the largest of these (the first rows'
+        // way in, too: M is below everything)
+        const double to = m - M[j] > kSlack ? m : M[j], sc = exp2_fast(M[j] - to);
+        s[j] *= sc;
+        s2[j] *= sc * sc;
+        M[j] = to;
+      }
+#pragma unroll
+      for (int t = 0; t < X::kRT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double e = exp2_fast(p[t][i] - M[j]);
+          s[j] += e;
+          s2[j] = fma(e, e, s2[j]);
+        }
+    }
+  }
+  // merge: 16 partials per point in LDS (over the rows' buffer), wavefront by
+  // wavefront and lane group by lane group
+  __syncthreads();
+  XPart *part = reinterpret_cast<XPart *>(sh);
+#pragma unroll
+  for (int j = 0; j < T; ++j)
+    part[w.part * (T * 16) + j * 16 + (w.lane & 15)] = XPart{M[j], s[j], s2[j]};
+  __syncthreads();
+  const int pt = w.pt0 + (int)threadIdx.x;
+  if (threadIdx.x < T * 16 && pt < a.npoints) {
+    XPart o{-DBL_MAX, 0.0, 0.0};
+#pragma unroll 2
+    for (int k = 0; k < 16; ++k) o.M = fmax(o.M, part[k * (T * 16) + threadIdx.x].M);
+#pragma unroll 2
+    for (int k = 0; k < 16; ++k) {
+      const XPart q = part[k * (T * 16) + threadIdx.x];
+      if (q.s == 0.0) continue;
+      const double sc = exp2_any(q.M - o.M);
+      o.s += q.s * sc;
+      o.s2 += q.s2 * sc * sc;
+    }
+    work[(size_t)pt * a.nchunks + w.chunk] = o;
+  }
+}
+
+__device__ inline double wave_max(double v) {
+  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, kWave));
+  return v;
+}
+__device__ inline double wave_add(double v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  return v;
+}
+
+// One wavefront per point: lanes take the chunks in turn, then a butterfly
+// (a thread per point walking its chunks took 63 us for one point on 1e5
+// genealogies and 160 us for 4096 on 1e6).
+__global__ __launch_bounds__(256) void jointp_exact_final(LArgs a, const XPart *work, double *out,
+                                                          double *ess) {
+  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  if (pt >= a.npoints) return;
+  const XPart *w = work + (size_t)pt * a.nchunks;
+  double M = -DBL_MAX;
+  for (int c = lane; c < a.nchunks; c += kWave) M = fmax(M, w[c].M);
+  M = wave_max(M);
+  double s = 0.0, s2 = 0.0;
+  for (int c = lane; c < a.nchunks; c += kWave) {
+    if (w[c].s == 0.0) continue;
+    const double sc = exp2_any(w[c].M - M);
+    s += w[c].s * sc;
+    s2 += w[c].s2 * sc * sc;
+  }
+  s = wave_add(s);
+  s2 = wave_add(s2);
+  if (lane == 0) {
+    out[pt] = log((double)a.G) - (M * kLn2 + log(s));
+    if (ess) ess[pt] = s * s / s2;
+  }
 }
 
 // ---------------------------------------------------------- REF_COMPAT --
@@ -263,165 +453,304 @@ __global__ void jointp_exact_final(LArgs a, const double *work, double *out, dou
 // whole final window, minus its smallest member when nothing outside the
 // window was kept and the window holds more than one value.
 //
-// pass 1: chunk maxima; pass 2: per chunk, the running maximum starts at
-// the maximum of the earlier chunks and each lane walks its rows in order;
-// pass 3: merge chunks in order and apply the list cap.
+// pass 1: chunk maxima; then, per point, the maxima of the chunks before
+// each one; pass 2: per chunk, the window sums, and whether a kept value
+// lies outside the window; final: the chunks merged and the list cap.
+//
+// A kept value's term is e^p / 10^maxz (the mantissa m 10^(z - maxz) of the
+// reference's eexp, utilities.cpp:1507-1539), taken here as 2^(p - maxz log2 10): the window, the list
+// cap and the ordering of the running maximum are the reference's, the term
+// itself differs from the degree-10 Taylor series of eexp by at most its
+// truncation, ~4e-10 relative, which moves the result by less than 1e-12
+// relative.
+constexpr double kWindow2 = 10.0 * kLog2E;
+constexpr double kLog2Of10 = 3.3219280948873623479;
 
-// Per (point, chunk) record of pass 2.
-struct RefPartial {
-  double sum, sum2;   // sum of scaled eexp terms (and squares) in the window
-  double minp, minterm;
-  int32_t cnt;        // values in the final window
-  int32_t outside;    // a kept value lies outside the final window
+// Per (point, chunk) record of pass 2: sums of the window's terms and of
+// their squares, its smallest value, its size, and whether a kept value
+// lies outside.
+struct RefPart {
+  double sum, sum2, minp;
+  int32_t cnt, outside;
 };
 
-// REF_COMPAT from the same compact records as EXACT, PTS points per lane.
-// Pass 1: chunk maxima.
-template <int NR, int PTS>
-__global__ __launch_bounds__(kXLanes) void jointp_ref_fast1(LArgs a, double *cmax) {
-  extern __shared__ double shrows[];
-  const int np = a.npsize + a.nmig;
-  double A[PTS][NR], F[PTS][NR], M[PTS];
-  int pt[PTS];
-#pragma unroll
-  for (int j = 0; j < PTS; ++j) {
-    pt[j] = blockIdx.x * (kXLanes * PTS) + j * kXLanes + threadIdx.x;
-    point_coef_compact<NR>(a, a.x + (size_t)(pt[j] < a.npoints ? pt[j] : 0) * np, A[j], F[j]);
-    M[j] = -DBL_MAX;
-  }
-  const int chunk = blockIdx.y;
-  const int gbeg = chunk * a.chunk_rows;
-  const int gend = min(a.G, gbeg + a.chunk_rows);
-  constexpr int RL = 1 + 2 * NR;
-  for (int g0 = gbeg; g0 < gend; g0 += a.stage) {
-    const int cnt = min(a.stage, gend - g0);
-    __syncthreads();
-    stage_compact(a, shrows, g0, cnt, NR);
-    __syncthreads();
-    for (int r = 0; r < cnt; ++r) {
-      const double *o = shrows + (size_t)r * RL;
-      double v[RL];
-#pragma unroll
-      for (int q = 0; q < RL; ++q) v[q] = o[q];
-#pragma unroll
-      for (int j = 0; j < PTS; ++j) M[j] = fmax(M[j], compact_term<NR>(v, A[j], F[j]));
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < PTS; ++j)
-    if (pt[j] < a.npoints) cmax[(size_t)pt[j] * a.nchunks + chunk] = M[j];
+// maxz: eexp's exponent of the largest term (10^z <= e^p < 10^(z + 1)) less 10
+__device__ inline int ref_maxz(double Mfin2) {
+  return (int)floor(Mfin2 * 0.30102999566398119521) - 10;
 }
 
-// Pass 2: per (point, chunk), the window sums.  A kept value's term is
-// e^p / 10^maxz (the reference's eexp mantissa m 10^(z - maxz)), taken here
-// as exp(p - maxz ln 10): the window, the list cap and the ordering of the
-// running maximum are the reference's, the term itself differs from the
-// degree-10 Taylor series of eexp by at most its truncation, ~4e-10
-// relative, which moves the result by less than 1e-12 relative.
-template <int NR, int PTS>
-__global__ __launch_bounds__(kXLanes) void jointp_ref_fast2(LArgs a, const double *cmax,
-                                                            RefPartial *part) {
-  extern __shared__ double shrows[];
-  const int np = a.npsize + a.nmig;
-  const int chunk = blockIdx.y;
-  double A[PTS][NR], F[PTS][NR], Mfin[PTS], run[PTS], sc[PTS];
-  RefPartial r[PTS];
-  int pt[PTS];
+template <int NR, int T>
+__global__ __launch_bounds__(kXLanes, 2) void jointp_ref_max(LArgs a, double *cmax) {
+  using X = XShape<NR>;
+  extern __shared__ double sh[];
+  double *shp = sh + X::kLds;
+  __shared__ int ptbad[T * 16];
+  const XPlace w = x_place<NR, T>(a);
+  stage_points<NR, T>(a, shp, ptbad, w.pt0);
+  PointFrag<NR> b[T];
+  double M[T];
 #pragma unroll
-  for (int j = 0; j < PTS; ++j) {
-    pt[j] = blockIdx.x * (kXLanes * PTS) + j * kXLanes + threadIdx.x;
-    const int ptc = pt[j] < a.npoints ? pt[j] : 0;
-    point_coef_compact<NR>(a, a.x + (size_t)ptc * np, A[j], F[j]);
-    const double *cm = cmax + (size_t)ptc * a.nchunks;
-    double mf = -DBL_MAX, ru = -DBL_MAX;
-    for (int c = 0; c < a.nchunks; ++c) {
-      mf = fmax(mf, cm[c]);
-      if (c < chunk) ru = fmax(ru, cm[c]);
-    }
-    Mfin[j] = mf;
-    run[j] = ru;
-    double mM;
-    int zM;
-    d_eexp(mf, &mM, &zM);
-    sc[j] = (double)(zM - 10) * 2.3025850929940456840;  // maxz ln 10
-    r[j] = RefPartial{0.0, 0.0, DBL_MAX, 0.0, 0, 0};
+  for (int j = 0; j < T; ++j) {
+    b[j].load(shp, j, w.lane);
+    M[j] = -DBL_MAX;
   }
-  const int gbeg = chunk * a.chunk_rows;
-  const int gend = min(a.G, gbeg + a.chunk_rows);
-  constexpr int RL = 1 + 2 * NR;
-  for (int g0 = gbeg; g0 < gend; g0 += a.stage) {
-    const int cnt = min(a.stage, gend - g0);
+  for (int g0 = w.gbeg; g0 < w.gend; g0 += X::kRows) {
+    const int cnt = min(X::kRows, w.gend - g0);
     __syncthreads();
-    stage_compact(a, shrows, g0, cnt, NR);
+    stage_rows<NR>(a, sh, g0, cnt);
     __syncthreads();
-    for (int rr = 0; rr < cnt; ++rr) {
-      const double *o = shrows + (size_t)rr * RL;
-      double v[RL];
+    RowFrag<NR> r;
+    r.load(sh, w.wave, w.lane);
 #pragma unroll
-      for (int q = 0; q < RL; ++q) v[q] = o[q];
-      const int g = g0 + rr;
+    for (int j = 0; j < T; ++j) {
+      dvec4 p[X::kRT];
+      terms<NR>(r, b[j], p);
+      if (cnt == X::kRows) {
+        M[j] = fmax(M[j], largest<NR>(p));
+      } else {
 #pragma unroll
-      for (int j = 0; j < PTS; ++j) {
-        const double p = compact_term<NR>(v, A[j], F[j]);
-        const bool kept = (g == 0) || (run[j] - p < 10);
-        if (kept && p > run[j]) run[j] = p;
-        if (Mfin[j] - p < 10) {
-          const double term = exp(p - sc[j]);
-          r[j].sum += term;
-          r[j].sum2 += term * term;
-          r[j].cnt += 1;
-          if (p < r[j].minp) {
-            r[j].minp = p;
-            r[j].minterm = term;
+        for (int t = 0; t < X::kRT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            M[j] = fmax(M[j], w.row0 + t * 16 + i < cnt ? p[t][i] : -DBL_MAX);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < T; ++j) sh[w.part * (T * 16) + j * 16 + (w.lane & 15)] = M[j];
+  __syncthreads();
+  const int pt = w.pt0 + (int)threadIdx.x;
+  if (threadIdx.x < T * 16 && pt < a.npoints) {
+    double m = -DBL_MAX;
+#pragma unroll 2
+    for (int k = 0; k < 16; ++k) m = fmax(m, sh[k * (T * 16) + threadIdx.x]);
+    cmax[(size_t)pt * a.nchunks + w.chunk] = m;
+  }
+}
+
+// The log2 term of one point (its parameters x) for one table row.
+__device__ inline double one_term(const LArgs &a, const float *g, const double *x) {
+  const JointLayout L = joint_layout(a.npsize, a.nmig);
+  double p;
+  if (a.npops == 2) {
+    p = -(double)g[L.probgp];
+  } else {
+    double t = 0.0;
+    if (a.modeltype == 1)
+      for (int i = 0; i < a.npsize; ++i) t += (double)g[L.qip + i];
+    else
+      for (int i = 0; i < a.nmig; ++i) t += (double)g[L.mip + i];
+    p = -t;
+  }
+  for (int i = a.r0; i < a.r1; ++i) {
+    if (i < a.npsize) {
+      const double A = (a.modeltype == 0 || a.modeltype == 1) ? kLn2 - log(x[i]) : 0.0;
+      p += (double)g[L.ccp + i] * A - (double)g[L.hccp + i] - 2.0 * (double)g[L.fcp + i] / x[i];
+    } else {
+      p += (double)g[L.mcp + i - a.npsize] * log(x[i]) - (double)g[L.fmp + i - a.npsize] * x[i];
+    }
+  }
+  return p * kLog2E;
+}
+
+// Per point, cmax[c] becomes the maximum over the chunks before c, and mfin
+// the maximum over all: one wavefront per point, 64 chunks at a time.  A
+// point whose first value (always kept) lies outside the final window needs
+// no further search for one: its cmax[c] are the final maximum.
+__global__ __launch_bounds__(256) void jointp_ref_prefix(LArgs a, double *cmax, double *mfin) {
+  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  if (pt >= a.npoints) return;
+  double *cm = cmax + (size_t)pt * a.nchunks;
+  const double first = one_term(a, a.rows, a.x + (size_t)pt * (a.npsize + a.nmig));
+  double before = -DBL_MAX;
+  for (int c0 = 0; c0 < a.nchunks; c0 += kWave) {
+    const int c = c0 + lane;
+    double v = c < a.nchunks ? cm[c] : -DBL_MAX;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const double o = __shfl_up(v, off, kWave);
+      if (lane >= off) v = fmax(v, o);
+    }
+    const double up = __shfl_up(v, 1, kWave);
+    if (c < a.nchunks) cm[c] = lane ? fmax(before, up) : before;
+    before = fmax(before, __shfl(v, kWave - 1, kWave));
+  }
+  if (lane == 0) mfin[pt] = before;
+  if (before - first >= kWindow2 + 1.0)  // clear of rounding: the kernel takes its own first value
+    for (int c = lane; c < a.nchunks; c += kWave) cm[c] = before;
+}
+
+template <int NR, int T>
+__global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const double *before,
+                                                             const double *mfin, RefPart *part) {
+  using X = XShape<NR>;
+  extern __shared__ double sh[];
+  double *shp = sh + X::kLds;
+  __shared__ int ptbad[T * 16];
+  __shared__ double smax[16][16], wmax[4][16];
+  const XPlace w = x_place<NR, T>(a);
+  stage_points<NR, T>(a, shp, ptbad, w.pt0);
+  PointFrag<NR> b[T];
+  double run[T], Mf[T], sc[T], seen[T];
+  RefPart o[T];
+  bool open = false;
+#pragma unroll
+  for (int j = 0; j < T; ++j) {
+    b[j].load(shp, j, w.lane);
+    const int pt = min(w.pt0 + j * 16 + (w.lane & 15), a.npoints - 1);
+    run[j] = before[(size_t)pt * a.nchunks + w.chunk];
+    Mf[j] = mfin[pt];
+    sc[j] = (double)ref_maxz(Mf[j]) * kLog2Of10;
+    seen[j] = -DBL_MAX;
+    o[j] = RefPart{0.0, 0.0, DBL_MAX, 0, 0};
+    open = open || run[j] < Mf[j];
+  }
+  // A kept value outside the final window lies within the window of a
+  // running maximum below the final one: once that is the final one (run =
+  // Mf, also set for points whose first value lies outside) there is none.
+  const bool look = __syncthreads_or(open) != 0;
+  for (int g0 = w.gbeg; g0 < w.gend; g0 += X::kRows) {
+    const int cnt = min(X::kRows, w.gend - g0);
+    __syncthreads();
+    stage_rows<NR>(a, sh, g0, cnt);
+    __syncthreads();
+    RowFrag<NR> r;
+    r.load(sh, w.wave, w.lane);
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      dvec4 p[X::kRT];
+      terms<NR>(r, b[j], p);
+      if (g0 == 0 && w.part == 0 && !(Mf[j] - p[0][0] < kWindow2)) o[j].outside = 1;
+      if (look) {
+        // candidates: within the window of the maximum before the chunk
+        bool cand = false;
+#pragma unroll
+        for (int t = 0; t < X::kRT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            cand = cand || (w.row0 + t * 16 + i < cnt && run[j] - p[t][i] < kWindow2 &&
+                            !(Mf[j] - p[t][i] < kWindow2));
+        if (__syncthreads_or(cand && !o[j].outside)) {
+          // with the running maximum before each value: the earlier chunks
+          // (run), the earlier stages (seen), the earlier wavefronts of this
+          // stage, the earlier tiles and lane groups of this wavefront
+          double m = -DBL_MAX;
+#pragma unroll 1
+          for (int x = 0; x < 4 * X::kRT; ++x)
+            if (w.row0 + x / 4 * 16 + x % 4 < cnt) m = fmax(m, pick<NR>(p, x));
+          m = fmax(m, __shfl_xor(m, 16, kWave));
+          m = fmax(m, __shfl_xor(m, 32, kWave));
+          if (w.lane < 16) wmax[w.wave][w.lane] = m;
+          smax[w.part][w.lane & 15] = seen[j];
+          __syncthreads();
+          double ru = run[j];
+#pragma unroll 1
+          for (int k = 0; k < 16; ++k) ru = fmax(ru, smax[k][w.lane & 15]);
+#pragma unroll 1
+          for (int k = 0; k < w.wave; ++k) ru = fmax(ru, wmax[k][w.lane & 15]);
+#pragma unroll 1
+          for (int t = 0; t < X::kRT; ++t) {
+            const int row = w.row0 + t * 16;
+            double m4 = -DBL_MAX;
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i)
+              if (row + i < cnt) m4 = fmax(m4, pick<NR>(p, 4 * t + i));
+            double st = ru;  // with the lane groups before this one
+#pragma unroll 1
+            for (int q = 0; q < 4; ++q) {
+              const double mq = __shfl(m4, q * 16 + (w.lane & 15), kWave);
+              if (q < (w.lane >> 4)) st = fmax(st, mq);
+              ru = fmax(ru, mq);
+            }
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i) {
+              if (row + i >= cnt) continue;
+              const double v = pick<NR>(p, 4 * t + i);
+              const bool kept = st - v < kWindow2;
+              if (kept && !(Mf[j] - v < kWindow2)) o[j].outside = 1;
+              if (kept && v > st) st = v;
+            }
           }
-        } else if (kept) {
-          r[j].outside = 1;
+          __syncthreads();  // smax and wmax are written again for the next tile
+        }
+#pragma unroll
+        for (int t = 0; t < X::kRT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            seen[j] = fmax(seen[j], w.row0 + t * 16 + i < cnt ? p[t][i] : -DBL_MAX);
+      }
+      // most values lie outside the window and cost no exp
+#pragma unroll
+      for (int t = 0; t < X::kRT; ++t) {
+        const int row = w.row0 + t * 16;
+        const double lo = Mf[j] - fmax(fmax(p[t][0], p[t][1]), fmax(p[t][2], p[t][3]));
+        if (!__any(lo < kWindow2)) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double v = p[t][i];
+          const bool in = row + i < cnt && Mf[j] - v < kWindow2;
+          const double e = in ? exp2_fast(v - sc[j]) : 0.0;
+          o[j].sum += e;
+          o[j].sum2 = fma(e, e, o[j].sum2);
+          o[j].cnt += in ? 1 : 0;
+          o[j].minp = fmin(o[j].minp, in ? v : DBL_MAX);
         }
       }
     }
   }
+  __syncthreads();
+  RefPart *lp = reinterpret_cast<RefPart *>(sh);
 #pragma unroll
-  for (int j = 0; j < PTS; ++j)
-    if (pt[j] < a.npoints) part[(size_t)pt[j] * a.nchunks + chunk] = r[j];
+  for (int j = 0; j < T; ++j)
+    lp[w.part * (T * 16) + j * 16 + (w.lane & 15)] = o[j];
+  __syncthreads();
+  const int pt = w.pt0 + (int)threadIdx.x;
+  if (threadIdx.x < T * 16 && pt < a.npoints) {
+    RefPart s{0.0, 0.0, DBL_MAX, 0, 0};
+#pragma unroll 2
+    for (int k = 0; k < 16; ++k) {
+      const RefPart q = lp[k * (T * 16) + threadIdx.x];
+      s.sum += q.sum;
+      s.sum2 += q.sum2;
+      s.minp = fmin(s.minp, q.minp);
+      s.cnt += q.cnt;
+      s.outside |= q.outside;
+    }
+    part[(size_t)pt * a.nchunks + w.chunk] = s;
+  }
 }
 
-template <int NR>
-hipError_t launch_ref_fast(const LArgs &a, dim3 grid_y, size_t lds, hipStream_t st,
-                           double *cmax, RefPartial *part) {
-  constexpr int PTS = NR <= 8 ? 2 : 1;
-  const dim3 grid((a.npoints + kXLanes * PTS - 1) / (kXLanes * PTS), grid_y.y);
-  hipLaunchKernelGGL((jointp_ref_fast1<NR, PTS>), grid, dim3(kXLanes), lds, st, a, cmax);
-  hipLaunchKernelGGL((jointp_ref_fast2<NR, PTS>), grid, dim3(kXLanes), lds, st, a, cmax, part);
-  return hipSuccess;
-}
-
-__global__ void jointp_ref_final(LArgs a, const double *cmax, const RefPartial *part,
-                                 double *out, double *ess) {
-  const int pt = blockIdx.x * blockDim.x + threadIdx.x;
+// One wavefront per point.
+__global__ __launch_bounds__(256) void jointp_ref_final(LArgs a, const double *mfin,
+                                                        const RefPart *part, double *out,
+                                                        double *ess) {
+  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
   if (pt >= a.npoints) return;
-  const RefPartial *P = part + (size_t)pt * a.nchunks;
-  const double *cm = cmax + (size_t)pt * a.nchunks;
-  double Mfin = -DBL_MAX;
-  for (int c = 0; c < a.nchunks; ++c) Mfin = fmax(Mfin, cm[c]);
-  double mM;
-  int zM;
-  d_eexp(Mfin, &mM, &zM);
-  const int maxz = zM - 10;
-  double sum = 0.0, sum2 = 0.0, minp = DBL_MAX, minterm = 0.0;
+  const RefPart *P = part + (size_t)pt * a.nchunks;
+  const int maxz = ref_maxz(mfin[pt]);
+  double sum = 0.0, sum2 = 0.0, minp = DBL_MAX;
   int cnt = 0, outside = 0;
-  for (int c = 0; c < a.nchunks; ++c) {
+  for (int c = lane; c < a.nchunks; c += kWave) {
     sum += P[c].sum;
     sum2 += P[c].sum2;
+    minp = fmin(minp, P[c].minp);
     cnt += P[c].cnt;
     outside |= P[c].outside;
-    if (P[c].cnt > 0 && P[c].minp < minp) {
-      minp = P[c].minp;
-      minterm = P[c].minterm;
-    }
   }
+  sum = wave_add(sum);
+  sum2 = wave_add(sum2);
+  minp = -wave_max(-minp);
+  for (int off = 32; off > 0; off >>= 1) {
+    cnt += __shfl_xor(cnt, off, kWave);
+    outside |= __shfl_xor(outside, off, kWave);
+  }
+  if (lane != 0) return;
   if (!outside && cnt > 1) {  // the list cap drops the smallest kept value
-    sum -= minterm;
-    sum2 -= minterm * minterm;
+    const double e = exp2_fast(minp - (double)maxz * kLog2Of10);
+    sum -= e;
+    sum2 -= e * e;
   }
   out[pt] = log((double)a.G) - (log(sum) + maxz * 2.3025850929940456840);
   if (ess) ess[pt] = sum * sum / sum2;
@@ -444,67 +773,89 @@ static void chunking(const LTable &t, int npoints, int *nchunks, int *chunk_rows
   *nchunks = (t.G + rows - 1) / rows;
 }
 
-size_t jointp_lds_bytes(const LTable &t) { return (size_t)stage_of(t) * t.K * 8; }
-
-// Compact records of the fast EXACT kernel: stage_of(t) rows of at most
-// 1 + 2 * 16 doubles.
-static size_t exact_lds_bytes(const LTable &t, int nr) {
-  return (size_t)stage_of(t) * xrec_len(nr) * 8;
-}
-
+// Work area: per point and chunk of the table a maximum and a partial, as
+// many chunks as `chunking` makes (the kernels' own chunks are no smaller).
 size_t jointp_work_bytes(const LTable &t, int npoints) {
   int nc, cr;
   chunking(t, npoints, &nc, &cr);
-  return (size_t)npoints * nc * (sizeof(double) + sizeof(RefPartial)) + 64;
+  return (size_t)npoints * nc * 48 + 64;
+}
+
+template <int NR, int T>
+static void x_grid(const LArgs &a, dim3 *grid, size_t *lds) {
+  using X = XShape<NR>;
+  *grid = dim3((a.npoints + 16 * T - 1) / (16 * T), a.nchunks);
+  *lds = std::max((size_t)(X::kLds + T * 16 * X::kKP) * 8,
+                  (size_t)16 * T * 16 * std::max(sizeof(XPart), sizeof(RefPart)));
+}
+
+// T tiles of points per workgroup, TS in the window sums (more registers a
+// tile).
+template <int NR, int T, int TS>
+static void launch_tiles(const LArgs &a, int mode, double *work, double *out, double *ess,
+                         hipStream_t st) {
+  const dim3 per_point((a.npoints + 3) / 4);
+  dim3 grid;
+  size_t lds;
+  x_grid<NR, T>(a, &grid, &lds);
+  if (mode == IMA_LMODE_EXACT) {
+    XPart *part = reinterpret_cast<XPart *>(work);
+    hipLaunchKernelGGL((jointp_exact<NR, T>), grid, dim3(kXLanes), lds, st, a, part);
+    hipLaunchKernelGGL(jointp_exact_final, per_point, dim3(256), 0, st, a, part, out, ess);
+  } else {
+    double *cmax = work, *mfin = cmax + (size_t)a.npoints * a.nchunks;
+    RefPart *part = reinterpret_cast<RefPart *>(mfin + a.npoints);
+    hipLaunchKernelGGL((jointp_ref_max<NR, T>), grid, dim3(kXLanes), lds, st, a, cmax);
+    hipLaunchKernelGGL(jointp_ref_prefix, per_point, dim3(256), 0, st, a, cmax, mfin);
+    x_grid<NR, TS>(a, &grid, &lds);
+    hipLaunchKernelGGL((jointp_ref_sum<NR, TS>), grid, dim3(kXLanes), lds, st, a, cmax, mfin,
+                       part);
+    hipLaunchKernelGGL(jointp_ref_final, per_point, dim3(256), 0, st, a, mfin, part, out, ess);
+  }
+}
+
+// Rows per chunk: chunking's, in whole stages.  Points per workgroup: a
+// workgroup stages each row once for all its tiles, so four tiles (two above
+// 8 parameters, for registers) as soon as they leave about a workgroup per
+// CU (256 points on 1e6 genealogies: 432 us with one tile, 317 with four;
+// 64 points: 134 and 112), and twice as many, at two workgroups a CU, once
+// there are several rounds of them (4096 points, 8 parameters: 6.5 and 5.1
+// ms; 500 points: 0.59 and 0.83 ms).  The values do not depend on it.
+constexpr int kMidGrid = 200, kWideGrid = 1024;
+
+template <int NR>
+static void launch_nr(LArgs a, int mode, double *work, double *out, double *ess, hipStream_t st) {
+  constexpr int kRows = XShape<NR>::kRows, kMid = NR <= 8 ? 4 : 2, kWide = 2 * kMid;
+  a.chunk_rows = (a.chunk_rows + kRows - 1) / kRows * kRows;
+  a.nchunks = (a.G + a.chunk_rows - 1) / a.chunk_rows;
+  auto groups = [&](int tiles) {
+    return (int64_t)((a.npoints + 16 * tiles - 1) / (16 * tiles)) * a.nchunks;
+  };
+  if (groups(kWide) >= kWideGrid)
+    launch_tiles<NR, kWide, kMid>(a, mode, work, out, ess, st);
+  else if (a.npoints > 16 * (kMid - 1) && groups(kMid) >= kMidGrid)
+    launch_tiles<NR, kMid, kMid>(a, mode, work, out, ess, st);
+  else
+    launch_tiles<NR, 1, 1>(a, mode, work, out, ess, st);
 }
 
 hipError_t launch_jointp(const LTable &t, const double *x, int npoints, int modeltype,
                          int r0, int r1, int mode, double *work, size_t work_bytes,
                          double *out, double *ess, hipStream_t st) {
   if (npoints == 0) return hipSuccess;
-  LArgs a{t.rows, t.G, t.K, t.npsize, t.nmig, t.npops, modeltype, r0, r1, x, npoints, 0, 0,
-          stage_of(t)};
+  LArgs a{t.rows, t.G, t.K, t.npsize, t.nmig, t.npops, modeltype, r0, r1, x, npoints, 0, 0};
   chunking(t, npoints, &a.nchunks, &a.chunk_rows);
   if (jointp_work_bytes(t, npoints) > work_bytes) return hipErrorInvalidValue;
-  const dim3 grid((npoints + kLTile - 1) / kLTile, a.nchunks);
-  const size_t lds = jointp_lds_bytes(t);
-  const int fin_blocks = (npoints + 255) / 256;
-  if (mode == IMA_LMODE_EXACT) {
-    const int nr = r1 - r0;
-    const size_t xl = exact_lds_bytes(t, nr);
-    switch (nr) {
-#define IMA_XCASE(N) \
-  case N:            \
-    launch_exact_fast<N>(a, grid, xl, st, work); \
+  switch (r1 - r0) {
+#define IMA_NR(N) \
+  case N:         \
+    launch_nr<N>(a, mode, work, out, ess, st); \
     break;
-      IMA_XCASE(1) IMA_XCASE(2) IMA_XCASE(3) IMA_XCASE(4) IMA_XCASE(5) IMA_XCASE(6)
-      IMA_XCASE(7) IMA_XCASE(8) IMA_XCASE(9) IMA_XCASE(10) IMA_XCASE(11) IMA_XCASE(12)
-      IMA_XCASE(13) IMA_XCASE(14) IMA_XCASE(15) IMA_XCASE(16)
-#undef IMA_XCASE
-      default:
-        return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(jointp_exact_final, dim3(fin_blocks), dim3(256), 0, st, a, work, out,
-                       ess);
-  } else {
-    double *cmax = work;
-    RefPartial *part = reinterpret_cast<RefPartial *>(cmax + (size_t)npoints * a.nchunks);
-    const int nr = r1 - r0;
-    const size_t xl = exact_lds_bytes(t, nr);
-    switch (nr) {
-#define IMA_RCASE(N) \
-  case N:            \
-    launch_ref_fast<N>(a, grid, xl, st, cmax, part); \
-    break;
-      IMA_RCASE(1) IMA_RCASE(2) IMA_RCASE(3) IMA_RCASE(4) IMA_RCASE(5) IMA_RCASE(6)
-      IMA_RCASE(7) IMA_RCASE(8) IMA_RCASE(9) IMA_RCASE(10) IMA_RCASE(11) IMA_RCASE(12)
-      IMA_RCASE(13) IMA_RCASE(14) IMA_RCASE(15) IMA_RCASE(16)
-#undef IMA_RCASE
-      default:
-        return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(jointp_ref_final, dim3(fin_blocks), dim3(256), 0, st, a, cmax, part,
-                       out, ess);
+    IMA_NR(1) IMA_NR(2) IMA_NR(3) IMA_NR(4) IMA_NR(5) IMA_NR(6) IMA_NR(7) IMA_NR(8)
+    IMA_NR(9) IMA_NR(10) IMA_NR(11) IMA_NR(12) IMA_NR(13) IMA_NR(14) IMA_NR(15) IMA_NR(16)
+#undef IMA_NR
+    default:
+      return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
