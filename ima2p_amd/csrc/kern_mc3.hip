@@ -318,19 +318,6 @@ __device__ inline double readlane_d(double x, int l) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Entry r of the all-loci sums after replacing one genealogy's weights
-// (sum_subtract_treeinfo, ginfo.cpp:249-285): counts add the difference,
-// fc / fm subtract then add and stay >= 0, hcc subtracts then adds.
-__device__ inline double wsum_update(int r, int P, double all, double old, double nw) {
-  const int P2 = P * P, P3 = P2 * P;
-  if (r < P2) return all + (nw - old);
-  if (r < 2 * P2) return fmax(0.0, (all - old) + nw);
-  if (r < 3 * P2) return (all - old) + nw;
-  if (r < 3 * P2 + P3) return all + (nw - old);
-  if (r < 3 * P2 + 2 * P3) return fmax(0.0, (all - old) + nw);
-  return (all - old) + nw;
-}
-
 // Pointers into the dynamic LDS of the per-chain prior kernels (PriorLds).
 //   all[R]           the chain's all-loci sums
 //   qt/qf/qc[np]     committed integral, weight, count of every parameter
@@ -467,7 +454,7 @@ __device__ inline bool param_hit(const ModelView &md, int P, int npsize, int t,
 // left.  The loci are taken in groups of D:
 //  1. one wavefront per locus reads its likelihood, uniform and records,
 //     flags the entries its proposal changed and marks the parameters they
-//     feed (for group g+2 while group g is being decided);
+//     feed (for group g + 2 beside step 2 of group g);
 //  2. one wavefront per parameter evaluates, one lane per scenario, the
 //     parameter's sums and integral for every locus j of the group under
 //     every combination S of the decisions on loci 0..j-1 (2^D - 1 lanes),
@@ -480,72 +467,107 @@ __device__ inline bool param_hit(const ModelView &md, int P, int npsize, int t,
 //  4. the group's records are committed or restored while the next group
 //     runs step 2.
 // The decisions and sums are those of deciding the loci one at a time.
+//
+// Bound: latency, group after group.  Of a group's 13 us at three
+// populations (wall clock inside the kernel) 7 were step 2, 3.7 the fetch of
+// a later group behind it, 2 the sums' update; with every lane's addresses
+// kept over the loop the compiler had put 70 registers in scratch memory,
+// and a load of one waited for the stores of the commit.  With the fetch
+// beside step 2, the scratch gone, the entry masks walked by scalar tests
+// and the decisions of all scenarios taken at once and picked by a ballot a
+// group takes 10 us at three populations and 7 at two; the launch went from
+// 130 to 107 us (64 chains x 50 loci), 579 to 417 us (256 x 300, two
+// populations) and 179 to 145 us (32 x 40, four populations).
 
-// Step 1 for the loci [l0, l0 + nl) of chain c into buffer rows b0.., by
-// wavefronts w0.. of the workgroup.
-__device__ inline void prior_fetch(const MC3Dev &m, const ModelView &md, int npsize,
-                                   const PriorSh &sh, const PriorLds &Lz, int c, int l0,
-                                   int nl, int b0, int w0, uint64_t sweep) {
+// Step 1 for one locus: its records, likelihood and uniform from memory,
+// the records' first kRecRegs * 64 entries through registers.
+constexpr int kRecRegs = 3;
+struct LocusFetch {
+  double o[kRecRegs], n[kRecRegs], npd, pdg, lu;
+  int ok;
+};
+__device__ __forceinline__ void prior_load(const MC3Dev &m, int it, LocusFetch &f) {
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  const int R = m.R;
+  const double *wo = m.wrec + (int64_t)it * R, *wn = m.wnew + (int64_t)it * R;
+#pragma unroll
+  for (int k = 0; k < kRecRegs; ++k) {
+    const int r = min(lane + k * kWave, R - 1);
+    f.o[k] = wo[r];
+    f.n[k] = wn[r];
+  }
+  f.ok = m.status[it] == IMA_STATUS_OK && m.wstatus[it] == IMA_STATUS_OK;
+  f.npd = new_loglik(m, it);
+  f.pdg = m.pdg[it];
+}
+// ... and into buffer row `row`: the records, which entries differ, the
+// parameters they feed.
+__device__ __forceinline__ void prior_store(const MC3Dev &m, const ModelView &md, int npsize,
+                                            const PriorSh &sh, const PriorLds &Lz, int it, int row,
+                                            const LocusFetch &f, uint64_t sweep) {
   const int R = m.R, np = m.nparam, P = m.P;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int nwaves = blockDim.x / kWave;
-  for (int x = wave - w0; x < nl; x += nwaves - w0) {
-    if (x < 0) break;
-    const int it = c * m.L + l0 + x, row = b0 + x;
-    const double *wo = m.wrec + (int64_t)it * R, *wn = m.wnew + (int64_t)it * R;
-    for (int r = lane; r < R; r += kWave) {
-      const double o = wo[r], w = wn[r];
-      sh.dold[row * R + r] = o;
-      sh.dnew[row * R + r] = w;
-      sh.flag[row * R + r] = o != w ? 1 : 0;
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  double *dold = sh.dold + (size_t)row * R, *dnew = sh.dnew + (size_t)row * R;
+  int *flag = sh.flag + (size_t)row * R;
+#pragma unroll
+  for (int k = 0; k < kRecRegs; ++k) {
+    const int r = lane + k * kWave;
+    if (r < R) {
+      dold[r] = f.o[k];
+      dnew[r] = f.n[k];
+      flag[r] = f.o[k] != f.n[k] ? 1 : 0;
     }
+  }
+  for (int r = lane + kRecRegs * kWave; r < R; r += kWave) {  // models of 5 and more populations
+    const double o = m.wrec[(int64_t)it * R + r], w = m.wnew[(int64_t)it * R + r];
+    dold[r] = o;
+    dnew[r] = w;
+    flag[r] = o != w ? 1 : 0;
+  }
+  if (lane == 0) {
+    sh.ok[row] = f.ok;
+    sh.npd[row] = f.npd;
+    sh.pdg[row] = f.pdg;
+    PhiloxStream rr = item_rng(m, it, sweep, 1);
+    // the decision U < min(1, e^x) is taken as log U < x (and U < 1);
+    // +inf stands for U = 1.  A host proposal's Hastings term h moves to
+    // this side: log U - h < beta (dprobg + gbeta dpdg)
+    const double U = m.uhost ? m.uhost[it] : rr.uniform();
+    sh.U[row] = (U < 1.0 ? log(U) : INFINITY) - (m.hast ? m.hast[it] : 0.0);
+  }
+  wave_sync();
+  for (int t0 = 0; t0 < np; t0 += kWave) {
+    const int t = t0 + lane;
+    const bool hit = t < np && param_hit(md, P, npsize, t, flag);
+    const unsigned long long bal = __ballot(hit);
     if (lane == 0) {
-      sh.ok[row] = m.status[it] == IMA_STATUS_OK && m.wstatus[it] == IMA_STATUS_OK;
-      sh.npd[row] = new_loglik(m, it);
-      sh.pdg[row] = m.pdg[it];
-      PhiloxStream rr = item_rng(m, it, sweep, 1);
-      // the decision U < min(1, e^x) is taken as log U < x (and U < 1);
-      // +inf stands for U = 1.  A host proposal's Hastings term h moves to
-      // this side: log U - h < beta (dprobg + gbeta dpdg)
-      const double U = m.uhost ? m.uhost[it] : rr.uniform();
-      sh.U[row] = (U < 1.0 ? log(U) : INFINITY) - (m.hast ? m.hast[it] : 0.0);
-    }
-    wave_sync();
-    for (int t0 = 0; t0 < np; t0 += kWave) {
-      const int t = t0 + lane;
-      const bool hit = t < np && param_hit(md, P, npsize, t, sh.flag + row * R);
-      const unsigned long long bal = __ballot(hit);
-      if (lane == 0) {
-        sh.aff[row * Lz.aw + t0 / 32] = (uint32_t)bal;
-        if (t0 / 32 + 1 < Lz.aw) sh.aff[row * Lz.aw + t0 / 32 + 1] = (uint32_t)(bal >> 32);
-      }
+      sh.aff[row * Lz.aw + t0 / 32] = (uint32_t)bal;
+      if (t0 / 32 + 1 < Lz.aw) sh.aff[row * Lz.aw + t0 / 32 + 1] = (uint32_t)(bal >> 32);
     }
   }
 }
 
-// Step 4 for the loci [l0, l0 + nl) held in buffer rows b0.., by the
-// workgroup's wavefronts from the last one down.
-__device__ inline void prior_commit(const DeviceView &v, const MC3Dev &m, const PriorSh &sh,
-                                    int c, int l0, int nl, int b0) {
+// Step 4 for locus item `it`, held in buffer row `row`; one wavefront.
+__device__ __forceinline__ void prior_commit(const DeviceView &v, const MC3Dev &m,
+                                             const PriorSh &sh, int it, int row) {
   const int R = m.R;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int nwaves = blockDim.x / kWave;
-  for (int x = nwaves - 1 - wave; x < nl; x += nwaves) {
-    const int it = c * m.L + l0 + x, row = b0 + x;
-    const bool acc = sh.dec[row] != 0;
-    if (acc) {
-      double *wc = m.wrec + (int64_t)it * R;
-      for (int r = lane; r < R; r += kWave)
-        if (sh.flag[row * R + r]) wc[r] = sh.dnew[row * R + r];
-    }
-    if (lane == 0) {
-      if (acc)
-        m.pdg[it] = sh.npd[row];
-      else if (!m.host && !m.topo)
-        restore_item(v, m, it);
-      if (m.host || m.topo) m.idec[it] = acc ? 1 : 0;
-      m.acc[it] += acc ? 1u : 0u;
-    }
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  const bool acc = sh.dec[row] != 0;
+  if (acc) {
+    double *wc = m.wrec + (int64_t)it * R;
+    for (int r = lane; r < R; r += kWave)
+      if (sh.flag[row * R + r]) wc[r] = sh.dnew[row * R + r];
+  }
+  if (lane == 0) {
+    if (acc)
+      m.pdg[it] = sh.npd[row];
+    else if (!m.host && !m.topo)
+      restore_item(v, m, it);
+    if (m.host || m.topo) m.idec[it] = acc ? 1 : 0;
+    if (acc) atomicAdd(&m.acc[it], 1u);  // no wait for its value
   }
 }
 
@@ -573,20 +595,95 @@ __device__ void prior_accept(const DeviceView &v, const MC3Dev &m, int c, uint64
   const ModelView md = model_view(sh.mi, sh.mdl, mm);
   double probg = m.probg[c];
   const double beta = m.beta[c];
-  // the first two groups; later ones are fetched two ahead while wave 0
-  // decides (their rows are those of the group committed just before)
-  prior_fetch(m, md, mm.npsize, sh, Lz, c, 0, min(D, m.L), 0, 0, sweep);
-  if (D < m.L) prior_fetch(m, md, mm.npsize, sh, Lz, c, D, min(D, m.L - D), D, 0, sweep);
+  // the first two groups; later ones are fetched two ahead, beside the
+  // integrals, by the last wavefronts (those without a parameter, where
+  // there are any; fetched after the integrals, beside the decisions, the
+  // groups waited 2.3 of 13 us for it), each locus by the one that commits
+  // the locus whose row it takes
+  for (int x = wave; x < min(2 * D, m.L); x += nwaves) {
+    LocusFetch f;
+    prior_load(m, c * m.L + x, f);
+    prior_store(m, md, mm.npsize, sh, Lz, c * m.L + x, x, f, sweep);
+  }
+  const int fx = nwaves - 1 - wave;  // the locus of a group this wavefront fetches and commits
+  // the logs of the first two of this wavefront's parameters' bounds
+  const double lmax0 = wave < np ? pri_log(prior_param_bound(md, mm.npsize, wave)) : 0.0;
+  const double lmax1 =
+      wave + nwaves < np ? pri_log(prior_param_bound(md, mm.npsize, wave + nwaves)) : 0.0;
   __syncthreads();
   // which loci of the group change each entry (group 0 here, group g + 1
   // beside the sums' update of group g)
   auto entry_masks = [&](int r, int b, int n) {
-    int mk = 0;
-    for (int j = 0; j < n; ++j) mk |= (sh.flag[(b + j) * R + r] ? 1 : 0) << j;
+    int v[kSpecDepth], mk = 0;
+#pragma unroll
+    for (int j = 0; j < kSpecDepth; ++j) v[j] = sh.flag[(b + min(j, D - 1)) * R + r];
+#pragma unroll
+    for (int j = 0; j < kSpecDepth; ++j) mk |= (j < n && v[j] ? 1 : 0) << j;
     sh.fmk[r] = mk;
   };
   for (int r = threadIdx.x; r < R; r += blockDim.x) entry_masks(r, 0, min(D, m.L));
   __syncthreads();
+  // Entry e (the same in every lane) of the all-loci sums with the records of
+  // the loci in sel that changed it put in, in order.  Which loci changed it
+  // is scalar: the records of the others are not read.
+  auto entry = [&](int e, int b, uint32_t sel, auto put) -> double {
+    const uint32_t bits = __builtin_amdgcn_readfirstlane(sh.fmk[e]);
+    double val = sh.all[e];
+#pragma unroll
+    for (int i = 0; i < kSpecDepth; ++i) {
+      if (!((bits >> i) & 1)) continue;
+      const size_t at = (size_t)(b + i) * R + e;
+      const double u = put(val, sh.dold[at], sh.dnew[at]);
+      val = (sel >> i) & 1 ? u : val;
+    }
+    return val;
+  };
+  // bit i: locus i of the group in rows b.. marks parameter t
+  auto marks = [&](int t, int b, int n) -> uint32_t {
+    uint32_t a[kSpecDepth], mk = 0;
+#pragma unroll
+    for (int i = 0; i < kSpecDepth; ++i) a[i] = sh.aff[(b + min(i, D - 1)) * Lz.aw + t / 32];
+#pragma unroll
+    for (int i = 0; i < kSpecDepth; ++i) mk |= (i < n ? (a[i] >> (t % 32)) & 1u : 0u) << i;
+    return mk;
+  };
+  // (term, weight, count) of parameter t from (term, f, c) after the loci in
+  // use, in order, each with the values of its scenario under S
+  struct Fold {
+    double term, f;
+    int c;
+  };
+  auto fold = [&](int t, uint32_t use, int S, double term, double f, int c) -> Fold {
+    double t2[kSpecDepth], f2[kSpecDepth];
+    int c2[kSpecDepth];
+#pragma unroll
+    for (int i = 0; i < kSpecDepth; ++i) {
+      const int si = min((1 << i) - 1 + (S & ((1 << i) - 1)), W - 1);
+      t2[i] = sh.sterm[t * W + si];
+      f2[i] = sh.sf[t * W + si];
+      c2[i] = sh.sc[t * W + si];
+    }
+#pragma unroll
+    for (int i = 0; i < kSpecDepth; ++i) {
+      const bool on = (use >> i) & 1;
+      if (on && !(c2[i] == c && f2[i] == f)) term = t2[i];
+      f = on ? f2[i] : f;
+      c = on ? c2[i] : c;
+    }
+    return Fold{term, f, c};
+  };
+  // acc += v[t * W], t from t0 to t1 in order, eight reads in flight
+  auto ordered_add = [&](double &acc, const double *su, int stride, int t0, int t1) {
+    int t = t0;
+    for (; t + 8 <= t1; t += 8) {
+      double x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = su[(t + k) * stride];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc += x[k];
+    }
+    for (; t < t1; ++t) acc += su[t * stride];
+  };
   // np <= 64: each scenario's prior total is formed before the decisions
   // (one lane per scenario), and a decision reads it from LDS
   const bool regs = np <= kWave;
@@ -594,31 +691,74 @@ __device__ void prior_accept(const DeviceView &v, const MC3Dev &m, int c, uint64
   for (int l0 = 0, g = 0; l0 < m.L; l0 += D, ++g) {
     const int nl = min(D, m.L - l0), b0 = (g % 3) * D, nb0 = ((g + 2) % 3) * D;
     const int nnl = l0 + 2 * D < m.L ? min(D, m.L - l0 - 2 * D) : 0;  // group g + 2
+    // 4. for the previous group and 1. for group g + 2, over its rows
+    if (fx < max(pnl, nnl)) {
+      const int it = c * m.L + l0 + 2 * D + fx;
+      LocusFetch f;
+      if (fx < nnl) prior_load(m, it, f);
+      if (fx < pnl) prior_commit(v, m, sh, c * m.L + pl0 + fx, pb0 + fx);
+      if (fx < nnl) prior_store(m, md, mm.npsize, sh, Lz, it, nb0 + fx, f, sweep);
+    }
     // 2. one wavefront per parameter, one lane per (locus j, decisions S)
     for (int t = wave; t < np; t += nwaves) {
-      const int s = lane;
-      if (s < W - 1) {
-        const int j = 31 - __clz(s + 1);
-        const int S = s + 1 - (1 << j);
-        if (j < nl && sh.ok[b0 + j] &&
-            ((sh.aff[(b0 + j) * Lz.aw + t / 32] >> (t % 32)) & 1u)) {
-          // the accepted loci of S and locus j, in order, that changed entry e
-          const uint32_t sel = (uint32_t)S | (1u << j);
-          auto get = [&](int e) {
-            double val = sh.all[e];
-            for (uint32_t bits = (uint32_t)sh.fmk[e] & sel; bits; bits &= bits - 1) {
-              const int row = b0 + (__ffs(bits) - 1);
-              val = wsum_update(e, P, val, sh.dold[row * R + e], sh.dnew[row * R + e]);
-            }
-            return val;
+      // (what follows from the lane is worked out here again: kept over the
+      // loop it took the registers to scratch memory, whose loads then waited
+      // for the commit's stores)
+      int s = lane;
+      asm volatile("" : "+v"(s));
+      const int j = 31 - __clz(s + 1), S = s + 1 - (1 << j);
+      const bool mine = s < W - 1 && j < nl;
+      // loci of the group that mark t (the same in every lane)
+      const uint32_t tm = marks(t, b0, nl);
+      const double qt = sh.qt[t], qf = sh.qf[t];
+      const int qc = sh.qc[t];
+      if (tm == 0) {  // no scenario changes t
+        if (regs && mine) sh.su[t * W + s] = qt;
+        continue;
+      }
+      // the accepted loci of S and locus j, in order, that changed an entry
+      const uint32_t sel = (uint32_t)S | (1u << j);
+      int cc = qc;
+      double f = qf, term = qt;
+      if (mine && sh.ok[b0 + j] && ((tm >> j) & 1u)) {
+        double h = 0.0;
+        f = 0.0;
+        cc = 0;
+        // counts first: the integral's log Gamma is read while the weights
+        // are summed
+        auto count = [](double v, double o, double n) { return v + (n - o); };
+        double lga = 0.0;
+        if (t < mm.npsize) {
+          for (int w = md.theta_off[t]; w < md.theta_off[t + 1]; ++w)
+            cc += (int)entry(md.theta_wp[2 * w] * P + md.theta_wp[2 * w + 1], b0, sel, count);
+          lga = prior_param_lga(mm.npsize, t, cc, v.logfact);
+          for (int w = md.theta_off[t]; w < md.theta_off[t + 1]; ++w) {
+            const int e = md.theta_wp[2 * w] * P + md.theta_wp[2 * w + 1];
+            f += entry(P * P + e, b0, sel,
+                       [](double v, double o, double n) { return fmax(0.0, (v - o) + n); });
+            h += entry(2 * P * P + e, b0, sel,
+                       [](double v, double o, double n) { return (v - o) + n; });
+          }
+        } else {
+          const int x = t - mm.npsize, P2 = P * P, P3 = P2 * P;
+          auto at = [&](int w) {
+            return (md.mig_wp[3 * w] * P + md.mig_wp[3 * w + 1]) * P + md.mig_wp[3 * w + 2];
           };
-          int cc;
-          double f, h;
-          prior_param_sums_of(md, P, mm.npsize, t, get, &cc, &f, &h);
-          sh.sc[t * W + s] = cc;
-          sh.sf[t * W + s] = f;
-          sh.sterm[t * W + s] = prior_param_term(md, mm.npsize, t, cc, f, h, v.logfact);
+          for (int w = md.mig_off[x]; w < md.mig_off[x + 1]; ++w)
+            cc += (int)entry(3 * P2 + at(w), b0, sel, count);
+          lga = prior_param_lga(mm.npsize, t, cc, v.logfact);
+          for (int w = md.mig_off[x]; w < md.mig_off[x + 1]; ++w) {
+            const int e = at(w);
+            f += entry(3 * P2 + P3 + e, b0, sel,
+                       [](double v, double o, double n) { return fmax(0.0, (v - o) + n); });
+          }
         }
+        const double max = prior_param_bound(md, mm.npsize, t);
+        const double lmax = t == wave ? lmax0 : t == wave + nwaves ? lmax1 : pri_log(max);
+        term = prior_param_term_lga(mm.npsize, t, cc, f, h, lga, max, lmax);
+        sh.sc[t * W + s] = cc;
+        sh.sf[t * W + s] = f;
+        sh.sterm[t * W + s] = term;
       }
       if (regs) {
         // the term scenario (j, S) uses for parameter t: from the group's
@@ -627,60 +767,50 @@ __device__ void prior_accept(const DeviceView &v, const MC3Dev &m, int c, uint64
         // keeping the committed term when count and weight are unchanged
         // (update_gtree_common.cpp:1997-2006)
         wave_sync();  // the scenario values of this wavefront's lanes
-        if (s < W - 1) {
-          const int j = 31 - __clz(s + 1);
-          const int S = s + 1 - (1 << j);
-          if (j < nl) {
-            double term = sh.qt[t], f = sh.qf[t];
-            int cc = sh.qc[t];
-            for (int i = 0; i <= j; ++i) {
-              if (i < j && !((S >> i) & 1)) continue;
-              if (!((sh.aff[(b0 + i) * Lz.aw + t / 32] >> (t % 32)) & 1u)) continue;
-              const int si = i == j ? s : (1 << i) - 1 + (S & ((1 << i) - 1));
-              const int c2 = sh.sc[t * W + si];
-              const double f2 = sh.sf[t * W + si];
-              if (!(c2 == cc && f2 == f)) term = sh.sterm[t * W + si];
-              cc = c2;
-              f = f2;
-            }
-            sh.su[t * W + s] = term;
-          }
-        }
+        if (mine) sh.su[t * W + s] = fold(t, tm & sel, S, qt, qf, qc).term;
       }
     }
-    // 4. for the previous group (whose rows group g + 2 takes next)
-    prior_commit(v, m, sh, c, pl0, pnl, pb0);
     __syncthreads();
     if (wave == 0) {
       // 3. decisions in order
       int Smask = 0;
       if (regs) {
         // each scenario's prior total, the parameters in order (population
-        // sizes, then migration rates)
-        if (lane < W - 1 && 31 - __clz(lane + 1) < nl) {
+        // sizes, then migration rates), and its decision: every lane takes
+        // its own scenario's, the chain's path then picks one per locus
+        int s = lane;
+        asm volatile("" : "+v"(s));
+        const int j = 31 - __clz(s + 1), S = s + 1 - (1 << j);
+        const bool mine = s < W - 1 && j < nl;
+        double pn = 0.0;
+        if (mine) {
+          const double *su = sh.su + s;
           double q = 0.0, mg = 0.0;
-          for (int t = 0; t < mm.npsize; ++t) q += sh.su[t * W + lane];
-          for (int t = mm.npsize; t < np; ++t) mg += sh.su[t * W + lane];
-          sh.pns[lane] = q + mg;
-        }
-        double xU = 0.0, xd = 0.0;  // lane j: U and the likelihood change of locus j
-        int okm = 0;
-        for (int j = 0; j < nl; ++j) okm |= (sh.ok[b0 + j] ? 1 : 0) << j;
-        if (lane < nl) {
-          xU = sh.U[b0 + lane];  // log U
-          xd = m.gbeta * (sh.npd[b0 + lane] - sh.pdg[b0 + lane]);
+          ordered_add(q, su, W, 0, mm.npsize);
+          ordered_add(mg, su, W, mm.npsize, np);
+          pn = q + mg;
+          sh.pns[s] = pn;
         }
         wave_sync();
-        for (int j = 0; j < nl; ++j) {
-          if (!((okm >> j) & 1)) continue;
-          const double pn = sh.pns[(1 << j) - 1 + Smask];
-          const double x = beta * ((pn - probg) + readlane_d(xd, j));
-          const double lu = readlane_d(xU, j);
-          const bool acc = x != x ? lu != INFINITY : lu < x;
-          if (acc) {
-            probg = pn;
-            Smask |= 1 << j;
+        bool yes = false;
+        if (mine && sh.ok[b0 + j]) {
+          // the total before locus j: the last accepted locus' of S
+          double before = probg;
+          if (S) {
+            const int i = 31 - __clz(S);
+            before = sh.pns[(1 << i) - 1 + (S ^ (1 << i))];
           }
+          const double xd = m.gbeta * (sh.npd[b0 + j] - sh.pdg[b0 + j]);
+          const double lu = sh.U[b0 + j];  // log U
+          const double x = beta * ((pn - before) + xd);
+          yes = x != x ? lu != INFINITY : lu < x;
+        }
+        const uint64_t dec = __ballot(yes);
+        for (int k = 0; k < nl; ++k)
+          Smask |= (int)((dec >> ((1 << k) - 1 + Smask)) & 1) << k;
+        if (Smask) {
+          const int i = 31 - __clz(Smask);
+          probg = sh.pns[(1 << i) - 1 + (Smask ^ (1 << i))];
         }
         if (lane < nl) sh.dec[b0 + lane] = (Smask >> lane) & 1;
       } else {
@@ -725,21 +855,38 @@ __device__ void prior_accept(const DeviceView &v, const MC3Dev &m, int c, uint64
           wave_sync();
         }
       }
-    } else if (nnl > 0) {
-      // 1. group g + 2
-      prior_fetch(m, md, mm.npsize, sh, Lz, c, l0 + 2 * D, nnl, nb0, 1, sweep);
     }
     __syncthreads();
     // the accepted changes into the sums, in locus order per entry; the
     // next group's entry masks
     const int n1 = l0 + D < m.L ? min(D, m.L - l0 - D) : 0, b1 = ((g + 1) % 3) * D;
     int accm = 0;  // the group's accepted loci
-    for (int j = 0; j < nl; ++j) accm |= (sh.dec[b0 + j] ? 1 : 0) << j;
-    for (int r = threadIdx.x; r < R; r += blockDim.x) {
+    {
+      int v[kSpecDepth];
+#pragma unroll
+      for (int j = 0; j < kSpecDepth; ++j) v[j] = sh.dec[b0 + min(j, D - 1)];
+#pragma unroll
+      for (int j = 0; j < kSpecDepth; ++j) accm |= (j < nl && v[j] ? 1 : 0) << j;
+      accm = __builtin_amdgcn_readfirstlane(accm);
+    }
+    int r0 = threadIdx.x;
+    asm volatile("" : "+v"(r0));
+    for (int r = r0; r < R; r += blockDim.x) {
+      // sum_subtract_treeinfo (ginfo.cpp:249-285): counts add the
+      // difference, fc / fm subtract then add and stay >= 0, the rest
+      // subtract then add
+      const int P2 = P * P, P3 = P2 * P;
+      const bool count = r < P2 || (r >= 3 * P2 && r < 3 * P2 + P3);
+      const bool keep = !count && r != R - 1 && (r < 2 * P2 || r >= 3 * P2);  // fc, fm: >= 0
       double a = sh.all[r];
-      for (uint32_t bits = (uint32_t)(sh.fmk[r] & accm); bits; bits &= bits - 1) {
-        const int row = b0 + (__ffs(bits) - 1);
-        a = wsum_update(r, P, a, sh.dold[row * R + r], sh.dnew[row * R + r]);
+      const uint32_t bits = (uint32_t)(sh.fmk[r] & accm);
+#pragma unroll
+      for (int i = 0; i < kSpecDepth; ++i) {
+        if (!((accm >> i) & 1)) continue;  // scalar
+        const double o = sh.dold[(b0 + i) * R + r], n = sh.dnew[(b0 + i) * R + r];
+        const double d = (a - o) + n;
+        const double u = count ? a + (n - o) : keep ? fmax(0.0, d) : d;
+        a = (bits >> i) & 1 ? u : a;
       }
       sh.all[r] = a;
       entry_masks(r, b1, n1);
@@ -747,29 +894,20 @@ __device__ void prior_accept(const DeviceView &v, const MC3Dev &m, int c, uint64
     if (regs && wave == nwaves - 1 && lane < np) {
       // the committed (term, weight, count) of parameter t after the group:
       // the scenario rule over the accepted loci
-      const int t = lane, Smask = accm;
-      double term = sh.qt[t], f = sh.qf[t];
-      int cc = sh.qc[t];
-      for (int i = 0; i < nl; ++i) {
-        if (!((Smask >> i) & 1)) continue;
-        if (!((sh.aff[(b0 + i) * Lz.aw + t / 32] >> (t % 32)) & 1u)) continue;
-        const int si = (1 << i) - 1 + (Smask & ((1 << i) - 1));
-        const int c2 = sh.sc[t * W + si];
-        const double f2 = sh.sf[t * W + si];
-        if (!(c2 == cc && f2 == f)) term = sh.sterm[t * W + si];
-        cc = c2;
-        f = f2;
-      }
-      sh.qt[t] = term;
-      sh.qf[t] = f;
-      sh.qc[t] = cc;
+      int t = lane;
+      asm volatile("" : "+v"(t));
+      const Fold o = fold(t, marks(t, b0, nl) & (uint32_t)accm, accm, sh.qt[t], sh.qf[t],
+                          sh.qc[t]);
+      sh.qt[t] = o.term;
+      sh.qf[t] = o.f;
+      sh.qc[t] = o.c;
     }
     __syncthreads();
     pl0 = l0;
     pnl = nl;
     pb0 = b0;
   }
-  prior_commit(v, m, sh, c, pl0, pnl, pb0);
+  if (fx < pnl) prior_commit(v, m, sh, c * m.L + pl0 + fx, pb0 + fx);
   __syncthreads();
   if (threadIdx.x == 0) m.probg[c] = probg;
   for (int r = threadIdx.x; r < R; r += blockDim.x) m.wall[(int64_t)c * R + r] = sh.all[r];
