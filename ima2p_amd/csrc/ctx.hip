@@ -60,6 +60,18 @@ hipError_t reserve(DevBuf<T> &b, size_t n, bool keep = false, hipStream_t st = n
   return hipSuccess;
 }
 
+// reserve() of a per-edge array that keeps its contents: the part that is new
+// holds zeros, so edges nothing has written yet read as population 0 without
+// migrations.  The device's copy is the only one: a run rewrites it there.
+template <typename T>
+hipError_t reserve_zeroed(DevBuf<T> &b, size_t n, hipStream_t st) {
+  const size_t old = b.p ? b.n : 0;
+  hipError_t e = reserve(b, n, true, st);
+  if (e == hipSuccess && b.n > old)
+    e = hipMemsetAsync(b.p + old, 0, (b.n - old) * sizeof(T), st);
+  return e;
+}
+
 template <typename T>
 void release(DevBuf<T> &b) {
   if (b.p) hipFree(b.p);
@@ -399,6 +411,7 @@ void ima_ctx_destroy(ima_ctx *c) {
   release(c->d_nw_newt);
   release(c->d_mv_off);
   release(c->d_mv_cnt);
+  release(c->d_mv_time);
   release(c->d_models);
   release(c->d_mint);
   release(c->d_mdbl);
@@ -531,20 +544,11 @@ int ima_slots_alloc(ima_ctx *c, int count, const int32_t *locus_of, int *first) 
     c->progs += (size_t)s.n - 1;
     c->slots.push_back(s);
   }
-  c->up0.resize(c->nodes, -1);
-  c->pop.resize(c->nodes, 0);
-  c->mig_first.resize(c->nodes, 0);
-  c->mig_count.resize(c->nodes, 0);
-  c->up1.resize(c->nodes, -1);
-  c->down.resize(c->nodes, -1);
-  c->A.resize(c->nodes, 0);
-  c->time.resize(c->nodes, 0.0);
-  c->prog.resize(c->progs);
   HIPCHK(c, reserve(c->d_up0, c->nodes, true, c->stream));
-  HIPCHK(c, reserve(c->d_pop, c->nodes, true, c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_pop, c->nodes, c->stream));
   HIPCHK(c, reserve(c->d_up1, c->nodes, true, c->stream));
   HIPCHK(c, reserve(c->d_down, c->nodes, true, c->stream));
-  HIPCHK(c, reserve(c->d_A, c->nodes, true, c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_A, c->nodes, c->stream));
   HIPCHK(c, reserve(c->d_time, c->nodes, true, c->stream));
   HIPCHK(c, reserve(c->d_prog, c->progs + 1, true, c->stream));
   c->slots_meta_dirty = true;
@@ -559,11 +563,13 @@ int ima_slots_write(ima_ctx *c, int first, int count, const int32_t *up0, const 
     return fail(c, IMA_ERR_ARG, "slot range [%d,%d) out of range", first, first + count);
   if (count == 0) return IMA_OK;
   hipSetDevice(c->device);
-  size_t src = 0;
-  std::vector<int> need;
+  // The slots of a range are adjacent in the node arrays, in the order the
+  // caller's arrays hold them: those go to the device as they are.
+  size_t src = 0, pb = 0;
+  std::vector<int> need, depth(count);
   std::vector<ProgOp> ops;
   for (int i = 0; i < count; ++i) {
-    SlotMeta &s = c->slots[first + i];
+    const SlotMeta &s = c->slots[first + i];
     const int n = s.n, ne = 2 * n - 1;
     std::string why;
     if (!valid_tree(n, up0 + src, up1 + src, down + src, time + src, root[i], why))
@@ -574,36 +580,33 @@ int ima_slots_write(ima_ctx *c, int first, int count, const int32_t *up0, const 
         first + i < c->mc3.first + c->mc3.C * c->mc3.L && std::max(1, r) > c->mc3.hmax_slots)
       return fail(c, IMA_ERR_STATE, "slot %d: program depth %d exceeds the running sweep's %d",
                   first + i, r, c->mc3.hmax_slots);
-    std::copy(up0 + src, up0 + src + ne, c->up0.begin() + s.node_off);
-    std::copy(up1 + src, up1 + src + ne, c->up1.begin() + s.node_off);
-    std::copy(down + src, down + src + ne, c->down.begin() + s.node_off);
-    std::copy(time + src, time + src + ne, c->time.begin() + s.node_off);
-    if (A) std::copy(A + src, A + src + ne, c->A.begin() + s.node_off);
-    s.root = root[i];
-    ops.clear();
+    ops.resize(pb);
     emit(up0 + src, up1 + src, root[i], need, ops);
-    std::copy(ops.begin(), ops.end(), c->prog.begin() + s.prog_off);
-    s.nslots = std::max(1, r);
+    depth[i] = std::max(1, r);
     src += ne;
+    pb += (size_t)n - 1;
+  }
+  ops.resize(pb);
+  for (int i = 0; i < count; ++i) {
+    c->slots[first + i].root = root[i];
+    c->slots[first + i].nslots = depth[i];
   }
   const SlotMeta &s0 = c->slots[first];
-  const SlotMeta &s1 = c->slots[first + count - 1];
-  const size_t nb = s1.node_off + 2 * (size_t)s1.n - 1 - s0.node_off;
-  const size_t pb = s1.prog_off + (size_t)s1.n - 1 - s0.prog_off;
-  HIPCHK(c, hipMemcpyAsync(c->d_up0.p + s0.node_off, c->up0.data() + s0.node_off, nb * 4,
-                           hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_up1.p + s0.node_off, c->up1.data() + s0.node_off, nb * 4,
-                           hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_down.p + s0.node_off, c->down.data() + s0.node_off, nb * 4,
-                           hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_time.p + s0.node_off, c->time.data() + s0.node_off, nb * 8,
-                           hipMemcpyHostToDevice, c->stream));
+  const size_t nb = src;
+  HIPCHK(c, hipMemcpyAsync(c->d_up0.p + s0.node_off, up0, nb * 4, hipMemcpyHostToDevice,
+                           c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_up1.p + s0.node_off, up1, nb * 4, hipMemcpyHostToDevice,
+                           c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_down.p + s0.node_off, down, nb * 4, hipMemcpyHostToDevice,
+                           c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_time.p + s0.node_off, time, nb * 8, hipMemcpyHostToDevice,
+                           c->stream));
   if (A)
-    HIPCHK(c, hipMemcpyAsync(c->d_A.p + s0.node_off, c->A.data() + s0.node_off, nb * 4,
-                             hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_A.p + s0.node_off, A, nb * 4, hipMemcpyHostToDevice,
+                             c->stream));
   if (pb)
-    HIPCHK(c, hipMemcpyAsync(c->d_prog.p + s0.prog_off, c->prog.data() + s0.prog_off,
-                             pb * sizeof(ProgOp), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_prog.p + s0.prog_off, ops.data(), pb * sizeof(ProgOp),
+                             hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, upload_slot_meta_range(c, first, count));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return IMA_OK;
@@ -1793,20 +1796,28 @@ static int mc3_topo_mode(ima_ctx *c, bool on) {
     int first = 0;
     if ((rc = ima_slots_alloc(c, N, loci.data(), &first)) != IMA_OK) return rc;
     m.topo_first = first;
-    HIPCHK(c, reserve(c->d_mig_first, c->nodes, true, c->stream));
-    HIPCHK(c, reserve(c->d_mig_count, c->nodes, true, c->stream));
+    HIPCHK(c, reserve_zeroed(c->d_mig_first, c->nodes, c->stream));
+    HIPCHK(c, reserve_zeroed(c->d_mig_count, c->nodes, c->stream));
   }
   HIPCHK(c, reserve(m.thast, N));
   HIPCHK(c, reserve(m.titems, N));
   HIPCHK(c, reserve(m.tptw, N));
   std::vector<int2> ar(m.L, make_int2(1, 1000));
+  std::vector<int32_t> alleles;  // of the first chain
+  const int64_t a0 = c->slots[m.first].node_off;
+  if (m.ns) {
+    const SlotMeta &e = c->slots[m.first + m.L - 1];
+    alleles.resize(e.node_off + 2 * (size_t)e.n - 1 - a0);
+    HIPCHK(c, copy_now(c, alleles.data(), c->d_A.p + a0, alleles.size() * 4,
+                       hipMemcpyDeviceToHost));
+  }
   for (int l = 0; l < m.L; ++l) {
     const SlotMeta &s = c->slots[m.first + l];
     if (c->loci[s.locus].model != IMA_MODEL_SW) continue;
     int mn = 1000, mx = 0;
     for (int e = 0; e < s.n; ++e) {
-      mn = std::min(mn, c->A[s.node_off + e]);
-      mx = std::max(mx, c->A[s.node_off + e]);
+      mn = std::min(mn, alleles[s.node_off - a0 + e]);
+      mx = std::max(mx, alleles[s.node_off - a0 + e]);
     }
     ar[l] = make_int2(std::max(1, (mx + mn) / 2 - (mx - mn)), std::min(1000, (mx + mn) / 2 + (mx - mn)));
   }
@@ -1874,7 +1885,7 @@ static int mc3_topo_mode(ima_ctx *c, bool on) {
 
 // Gives slots[i] room for at least caps[i] migration events: the events of
 // each slot that needs more move to a new region at the end of the event
-// arrays (host mirror and device).
+// arrays.
 static int grow_mig_caps(ima_ctx *c, const int32_t *slots, const int32_t *caps, int n) {
   std::vector<int64_t> from, to;
   std::vector<int32_t> cnt;
@@ -1889,22 +1900,10 @@ static int grow_mig_caps(ima_ctx *c, const int32_t *slots, const int32_t *caps, 
     c->migs += (size_t)caps[i];
   }
   if (from.empty()) return IMA_OK;
-  c->mig_edge.resize(c->migs, 0);
-  c->mig_to.resize(c->migs, 0);
-  c->mig_time.resize(c->migs, 0.0);
-  for (size_t i = 0; i < from.size(); ++i) {
-    std::copy(c->mig_edge.begin() + from[i], c->mig_edge.begin() + from[i] + cnt[i],
-              c->mig_edge.begin() + to[i]);
-    std::copy(c->mig_to.begin() + from[i], c->mig_to.begin() + from[i] + cnt[i],
-              c->mig_to.begin() + to[i]);
-    std::copy(c->mig_time.begin() + from[i], c->mig_time.begin() + from[i] + cnt[i],
-              c->mig_time.begin() + to[i]);
-  }
   HIPCHK(c, reserve(c->d_mig_edge, c->migs + 1, true, c->stream));
   HIPCHK(c, reserve(c->d_mig_to, c->migs + 1, true, c->stream));
   HIPCHK(c, reserve(c->d_mig_time, c->migs + 1, true, c->stream));
-  // the device's events (their times may have moved since the host wrote
-  // them) follow to the new regions, one launch for every slot
+  // the events follow to the new regions, one launch for every slot
   const size_t m = from.size();
   HIPCHK(c, reserve(c->d_mv_off, 2 * m));
   HIPCHK(c, reserve(c->d_mv_cnt, m));
@@ -1912,34 +1911,10 @@ static int grow_mig_caps(ima_ctx *c, const int32_t *slots, const int32_t *caps, 
   HIPCHK(c, hipMemcpyAsync(c->d_mv_off.p + m, to.data(), m * 8, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->d_mv_cnt.p, cnt.data(), m * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, launch_move_events((int)m, c->d_mv_off.p, c->d_mv_off.p + m, c->d_mv_cnt.p,
-                               c->d_mig_edge.p, c->d_mig_to.p, c->d_mig_time.p, c->stream));
+                               c->d_mig_edge.p, c->d_mig_to.p, c->d_mig_time.p, c->d_mig_edge.p,
+                               c->d_mig_to.p, c->d_mig_time.p, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));  // the host arrays above are freed on return
   c->slots_meta_dirty = true;
-  return IMA_OK;
-}
-
-// The host mirror of the slots' populations, per-edge indexes and events,
-// uploaded (the NW update reads them on the device).
-static int nw_upload_slots(ima_ctx *c, const int32_t *slots, int nslots) {
-  HIPCHK(c, reserve(c->d_pop, c->nodes, true, c->stream));
-  for (int i = 0; i < nslots; ++i) {
-    const SlotMeta &s = c->slots[slots[i]];
-    const size_t ne = 2 * (size_t)s.n - 1;
-    HIPCHK(c, hipMemcpyAsync(c->d_pop.p + s.node_off, c->pop.data() + s.node_off, ne * 4,
-                             hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_first.p + s.node_off, c->mig_first.data() + s.node_off,
-                             ne * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_count.p + s.node_off, c->mig_count.data() + s.node_off,
-                             ne * 4, hipMemcpyHostToDevice, c->stream));
-    if (s.nmig) {
-      HIPCHK(c, hipMemcpyAsync(c->d_mig_edge.p + s.mig_off, c->mig_edge.data() + s.mig_off,
-                               (size_t)s.nmig * 4, hipMemcpyHostToDevice, c->stream));
-      HIPCHK(c, hipMemcpyAsync(c->d_mig_to.p + s.mig_off, c->mig_to.data() + s.mig_off,
-                               (size_t)s.nmig * 4, hipMemcpyHostToDevice, c->stream));
-      HIPCHK(c, hipMemcpyAsync(c->d_mig_time.p + s.mig_off, c->mig_time.data() + s.mig_off,
-                               (size_t)s.nmig * 8, hipMemcpyHostToDevice, c->stream));
-    }
-  }
   return IMA_OK;
 }
 
@@ -1959,41 +1934,17 @@ static int nw_reserve_backups(ima_ctx *c) {
   HIPCHK(c, reserve(c->d_nw_mto, c->migs + 1));
   HIPCHK(c, reserve(c->d_nw_mt, c->migs + 1));
   // per-edge migration indexes on the device for every slot
-  if (c->d_mig_first.n < c->nodes || c->d_mig_count.n < c->nodes) {
-    HIPCHK(c, reserve(c->d_mig_first, c->nodes, false, c->stream));
-    HIPCHK(c, reserve(c->d_mig_count, c->nodes, false, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_first.p, c->mig_first.data(), c->nodes * 4,
-                             hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_count.p, c->mig_count.data(), c->nodes * 4,
-                             hipMemcpyHostToDevice, c->stream));
-  }
+  HIPCHK(c, reserve_zeroed(c->d_mig_first, c->nodes, c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_mig_count, c->nodes, c->stream));
   return IMA_OK;
 }
 
-// The host mirror of slots whose populations and migrations the device
-// rewrote: slot records, populations, per-edge indexes and events.
-static int nw_sync_slots(ima_ctx *c, const int32_t *slots, int nslots) {
-  for (int i = 0; i < nslots; ++i) {
-    const int sl = slots[i];
-    HIPCHK(c, copy_now(c, &c->slots[sl], c->d_slots.p + sl, sizeof(SlotMeta),
-                       hipMemcpyDeviceToHost));
-    const SlotMeta &s = c->slots[sl];
-    const size_t ne = 2 * (size_t)s.n - 1;
-    HIPCHK(c, copy_now(c, c->pop.data() + s.node_off, c->d_pop.p + s.node_off, ne * 4,
-                       hipMemcpyDeviceToHost));
-    HIPCHK(c, copy_now(c, c->mig_first.data() + s.node_off, c->d_mig_first.p + s.node_off,
-                       ne * 4, hipMemcpyDeviceToHost));
-    HIPCHK(c, copy_now(c, c->mig_count.data() + s.node_off, c->d_mig_count.p + s.node_off,
-                       ne * 4, hipMemcpyDeviceToHost));
-    if (s.nmig) {
-      HIPCHK(c, copy_now(c, c->mig_edge.data() + s.mig_off, c->d_mig_edge.p + s.mig_off,
-                         (size_t)s.nmig * 4, hipMemcpyDeviceToHost));
-      HIPCHK(c, copy_now(c, c->mig_to.data() + s.mig_off, c->d_mig_to.p + s.mig_off,
-                         (size_t)s.nmig * 4, hipMemcpyDeviceToHost));
-      HIPCHK(c, copy_now(c, c->mig_time.data() + s.mig_off, c->d_mig_time.p + s.mig_off,
-                         (size_t)s.nmig * 8, hipMemcpyDeviceToHost));
-    }
-  }
+// The host's records of slots whose genealogies the device rewrote.
+static int sync_slot_meta(ima_ctx *c, const int32_t *slots, int nslots) {
+  for (int i = 0; i < nslots; ++i)
+    HIPCHK(c, hipMemcpyAsync(&c->slots[slots[i]], c->d_slots.p + slots[i], sizeof(SlotMeta),
+                             hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   return IMA_OK;
 }
 
@@ -2108,56 +2059,15 @@ static int mc3_nw_mode(ima_ctx *c, bool on) {
   return mc3_nw_buffers(c);
 }
 
-// After a run with the NW update: the host mirror of the chains' slot
-// records, populations, per-edge migration indexes and events follows the
-// device.
-static int mc3_nw_sync(ima_ctx *c) {
+// After a run that moves genealogies or migrations (IMA_MC3_TOPOLOGY,
+// IMA_MC3_NW) the host's records of the chains' slots (root, program depth,
+// event count) follow the device's.  The genealogies themselves are on the
+// device only: a copy of every chain's trees and events behind each run was
+// 17 of the 36 ms of ten sweeps on 256 chains x 300 loci.
+static int mc3_sync(ima_ctx *c) {
   auto &m = c->mc3;
-  const int N = m.C * m.L;
-  const SlotMeta &s0 = c->slots[m.first];
-  const SlotMeta &s1 = c->slots[m.first + N - 1];
-  const size_t nb = s1.node_off + 2 * (size_t)s1.n - 1 - s0.node_off;
-  const size_t o = s0.node_off;
-  HIPCHK(c, copy_now(c, c->slots.data() + m.first, c->d_slots.p + m.first, N * sizeof(SlotMeta),
-                     hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->pop.data() + o, c->d_pop.p + o, nb * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->mig_first.data() + o, c->d_mig_first.p + o, nb * 4,
-                     hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->mig_count.data() + o, c->d_mig_count.p + o, nb * 4,
-                     hipMemcpyDeviceToHost));
-  if (c->migs) {
-    HIPCHK(c, copy_now(c, c->mig_edge.data(), c->d_mig_edge.p, c->migs * 4,
-                       hipMemcpyDeviceToHost));
-    HIPCHK(c, copy_now(c, c->mig_to.data(), c->d_mig_to.p, c->migs * 4, hipMemcpyDeviceToHost));
-    HIPCHK(c, copy_now(c, c->mig_time.data(), c->d_mig_time.p, c->migs * 8,
-                       hipMemcpyDeviceToHost));
-  }
-  return IMA_OK;
-}
-
-// After a run with the device's own genealogy move: the host mirror of the
-// chains' slots follows the device (topologies, times, populations,
-// alleles, programs and slot records).
-static int mc3_topo_sync(ima_ctx *c) {
-  auto &m = c->mc3;
-  const int N = m.C * m.L;
-  const SlotMeta &s0 = c->slots[m.first];
-  const SlotMeta &s1 = c->slots[m.first + N - 1];
-  const size_t nb = s1.node_off + 2 * (size_t)s1.n - 1 - s0.node_off;
-  const size_t pb = s1.prog_off + (size_t)s1.n - 1 - s0.prog_off;
-  const size_t o = s0.node_off;
-  HIPCHK(c, copy_now(c, c->slots.data() + m.first, c->d_slots.p + m.first, N * sizeof(SlotMeta),
-                     hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->up0.data() + o, c->d_up0.p + o, nb * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->up1.data() + o, c->d_up1.p + o, nb * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->down.data() + o, c->d_down.p + o, nb * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->time.data() + o, c->d_time.p + o, nb * 8, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->pop.data() + o, c->d_pop.p + o, nb * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, copy_now(c, c->A.data() + o, c->d_A.p + o, nb * 4, hipMemcpyDeviceToHost));
-  if (pb)
-    HIPCHK(c, copy_now(c, c->prog.data() + s0.prog_off, c->d_prog.p + s0.prog_off,
-                       pb * sizeof(ProgOp), hipMemcpyDeviceToHost));
-  if (m.dev.mig_pool > 0) return mc3_nw_sync(c);  // the migrations the moves drew
+  HIPCHK(c, copy_now(c, c->slots.data() + m.first, c->d_slots.p + m.first,
+                     (size_t)m.C * m.L * sizeof(SlotMeta), hipMemcpyDeviceToHost));
   return IMA_OK;
 }
 
@@ -2312,9 +2222,8 @@ extern "C" {
 int ima_mc3_run(ima_ctx *c, int nsweeps, int flags) {
   int rc = mc3_run_async(c, nsweeps, flags);
   if (rc != IMA_OK) return rc;
+  if (c->mc3.dev.topo || c->mc3.dev.nw) return mc3_sync(c);
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (c->mc3.dev.topo) return mc3_topo_sync(c);
-  if (c->mc3.dev.nw) return mc3_nw_sync(c);
   return IMA_OK;
 }
 
@@ -2759,13 +2668,6 @@ int ima_mc3_decide(ima_ctx *c, int prop_first, const double *hastings, const dou
           d.mig_off = (int64_t)c->migs;
           d.mig_cap = cap;
           c->migs += (size_t)cap;
-          c->mig_edge.resize(c->migs, 0);
-          c->mig_to.resize(c->migs, 0);
-          c->mig_time.resize(c->migs, 0.0);
-          std::copy(c->mig_edge.begin() + old, c->mig_edge.begin() + old + d.nmig,
-                    c->mig_edge.begin() + d.mig_off);
-          std::copy(c->mig_to.begin() + old, c->mig_to.begin() + old + d.nmig,
-                    c->mig_to.begin() + d.mig_off);
           HIPCHK(c, reserve(c->d_mig_edge, c->migs + 1, true, c->stream));
           HIPCHK(c, reserve(c->d_mig_to, c->migs + 1, true, c->stream));
           HIPCHK(c, reserve(c->d_mig_time, c->migs + 1, true, c->stream));
@@ -2788,14 +2690,8 @@ int ima_mc3_decide(ima_ctx *c, int prop_first, const double *hastings, const dou
     return fail(c, IMA_ERR_SIZE, "a proposal has %d prior events", emax);
   // per-edge migration indexes of every slot on the device (slots allocated
   // after the last ima_slots_write_pops have none there yet)
-  if (c->d_mig_first.n < c->nodes || c->d_mig_count.n < c->nodes) {
-    HIPCHK(c, reserve(c->d_mig_first, c->nodes, false, c->stream));
-    HIPCHK(c, reserve(c->d_mig_count, c->nodes, false, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_first.p, c->mig_first.data(), c->nodes * 4,
-                             hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_count.p, c->mig_count.data(), c->nodes * 4,
-                             hipMemcpyHostToDevice, c->stream));
-  }
+  HIPCHK(c, reserve_zeroed(c->d_mig_first, c->nodes, c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_mig_count, c->nodes, c->stream));
   if (grew) {
     HIPCHK(c, reserve(m.mtbackup, c->migs + 1));
     m.dev.mtbackup = m.mtbackup.p;
@@ -2848,30 +2744,11 @@ int ima_mc3_decide(ima_ctx *c, int prop_first, const double *hastings, const dou
   std::vector<int32_t> dec(N);
   HIPCHK(c, copy_now(c, dec.data(), m.idec.p, (size_t)N * 4, hipMemcpyDeviceToHost));
   m.host_sweeps += 1;  // the device counter advanced with the decisions
-  // the host mirror of the chains' slots follows the device copy
+  // the host's records of the chains' slots follow the device's
   for (int i = 0; i < N; ++i) {
     if (!dec[i]) continue;
     SlotMeta &dst = c->slots[m.first + i];
     const SlotMeta &src = c->slots[prop_first + i];
-    const int64_t so = src.node_off, dn = dst.node_off, ne = 2 * (int64_t)src.n - 1;
-    std::copy(c->up0.begin() + so, c->up0.begin() + so + ne, c->up0.begin() + dn);
-    std::copy(c->up1.begin() + so, c->up1.begin() + so + ne, c->up1.begin() + dn);
-    std::copy(c->down.begin() + so, c->down.begin() + so + ne, c->down.begin() + dn);
-    std::copy(c->time.begin() + so, c->time.begin() + so + ne, c->time.begin() + dn);
-    std::copy(c->A.begin() + so, c->A.begin() + so + ne, c->A.begin() + dn);
-    std::copy(c->pop.begin() + so, c->pop.begin() + so + ne, c->pop.begin() + dn);
-    std::copy(c->mig_first.begin() + so, c->mig_first.begin() + so + ne, c->mig_first.begin() + dn);
-    std::copy(c->mig_count.begin() + so, c->mig_count.begin() + so + ne, c->mig_count.begin() + dn);
-    std::copy(c->prog.begin() + src.prog_off, c->prog.begin() + src.prog_off + src.n - 1,
-              c->prog.begin() + dst.prog_off);
-    if (src.nmig) {
-      std::copy(c->mig_edge.begin() + src.mig_off, c->mig_edge.begin() + src.mig_off + src.nmig,
-                c->mig_edge.begin() + dst.mig_off);
-      std::copy(c->mig_to.begin() + src.mig_off, c->mig_to.begin() + src.mig_off + src.nmig,
-                c->mig_to.begin() + dst.mig_off);
-      std::copy(c->mig_time.begin() + src.mig_off, c->mig_time.begin() + src.mig_off + src.nmig,
-                c->mig_time.begin() + dst.mig_off);
-    }
     dst.root = src.root;
     dst.nslots = src.nslots;
     dst.nmig = src.nmig;
@@ -3066,7 +2943,7 @@ int ima_slots_write_pops(ima_ctx *c, int first, int count, const int32_t *pop,
   hipSetDevice(c->device);
   size_t src = 0, msrc = 0;
   for (int i = 0; i < count; ++i) {
-    SlotMeta &s = c->slots[first + i];
+    const SlotMeta &s = c->slots[first + i];
     const LocusMeta &lm = c->loci[s.locus];
     if (lm.pmodel < 0) return fail(c, IMA_ERR_STATE, "slot %d: its locus has no population model", first + i);
     const int T = 2 * c->models[lm.pmodel].npops - 1, ne = 2 * s.n - 1;
@@ -3084,53 +2961,103 @@ int ima_slots_write_pops(ima_ctx *c, int first, int count, const int32_t *pop,
                     (mig_edge[q] == mig_edge[q - 1] && mig_time[q] < mig_time[q - 1])))
         return fail(c, IMA_ERR_ARG, "slot %d: migrations not sorted by edge then time", first + i);
     }
-    std::copy(pop + src, pop + src + ne, c->pop.begin() + s.node_off);
+    src += ne;
+    msrc += nmig[i];
+  }
+  // The slots of a range are adjacent in the node arrays.  Their event
+  // regions are too when this call made them (a slot keeps the region it has
+  // while its events fit), with some room behind each slot's events.
+  std::vector<int32_t> mfirst(src, 0), mcount(src, 0);
+  bool dense = true;
+  int64_t m0 = -1, mend = 0;
+  src = msrc = 0;
+  for (int i = 0; i < count; ++i) {
+    SlotMeta &s = c->slots[first + i];
     if (nmig[i] > s.mig_cap) {
       s.mig_cap = nmig[i] + nmig[i] / 2 + 4;
       s.mig_off = (int64_t)c->migs;
       c->migs += (size_t)s.mig_cap;
-      c->mig_edge.resize(c->migs, 0);
-      c->mig_to.resize(c->migs, 0);
-      c->mig_time.resize(c->migs, 0.0);
     }
     s.nmig = nmig[i];
-    std::fill(c->mig_count.begin() + s.node_off, c->mig_count.begin() + s.node_off + ne, 0);
-    std::fill(c->mig_first.begin() + s.node_off, c->mig_first.begin() + s.node_off + ne, 0);
     for (int j = nmig[i] - 1; j >= 0; --j) {
       const int e = mig_edge[msrc + j];
-      c->mig_first[s.node_off + e] = j;
-      c->mig_count[s.node_off + e] += 1;
+      mfirst[src + e] = j;
+      mcount[src + e] += 1;
     }
     if (nmig[i]) {
-      std::copy(mig_edge + msrc, mig_edge + msrc + nmig[i], c->mig_edge.begin() + s.mig_off);
-      std::copy(mig_to + msrc, mig_to + msrc + nmig[i], c->mig_to.begin() + s.mig_off);
-      std::copy(mig_time + msrc, mig_time + msrc + nmig[i], c->mig_time.begin() + s.mig_off);
+      if (m0 < 0) m0 = s.mig_off;
+      else dense = dense && s.mig_off == mend;
+      mend = s.mig_off + s.mig_cap;
     }
-    src += ne;
+    src += 2 * (size_t)s.n - 1;
     msrc += nmig[i];
   }
   const SlotMeta &s0 = c->slots[first];
-  const SlotMeta &s1 = c->slots[first + count - 1];
-  const size_t nb = s1.node_off + 2 * (size_t)s1.n - 1 - s0.node_off;
-  HIPCHK(c, reserve(c->d_pop, c->nodes, true, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_pop.p + s0.node_off, c->pop.data() + s0.node_off, nb * 4,
+  const size_t nb = src;
+  HIPCHK(c, reserve_zeroed(c->d_pop, c->nodes, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_pop.p + s0.node_off, pop, nb * 4, hipMemcpyHostToDevice,
+                           c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_mig_first, c->nodes, c->stream));
+  HIPCHK(c, reserve_zeroed(c->d_mig_count, c->nodes, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_mig_first.p + s0.node_off, mfirst.data(), nb * 4,
                            hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, reserve(c->d_mig_first, c->nodes, true, c->stream));
-  HIPCHK(c, reserve(c->d_mig_count, c->nodes, true, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_mig_first.p + s0.node_off, c->mig_first.data() + s0.node_off,
-                           nb * 4, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_mig_count.p + s0.node_off, c->mig_count.data() + s0.node_off,
-                           nb * 4, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_mig_count.p + s0.node_off, mcount.data(), nb * 4,
+                           hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, reserve(c->d_mig_edge, c->migs + 1, true, c->stream));
   HIPCHK(c, reserve(c->d_mig_to, c->migs + 1, true, c->stream));
   HIPCHK(c, reserve(c->d_mig_time, c->migs + 1, true, c->stream));
-  if (c->migs) {
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_edge.p, c->mig_edge.data(), c->migs * 4,
-                             hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_to.p, c->mig_to.data(), c->migs * 4,
-                             hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_mig_time.p, c->mig_time.data(), c->migs * 8,
-                             hipMemcpyHostToDevice, c->stream));
+  std::vector<int32_t> pe, pt, cnt;
+  std::vector<double> pm;
+  std::vector<int64_t> from, to;
+  if (m0 >= 0 && dense) {
+    // one block of regions: laid out here, one copy of each array (of one
+    // slot, as IMa2p's per-locus path writes them, just its events)
+    const size_t len = (size_t)(mend - m0);
+    pe.assign(len, 0);
+    pt.assign(len, 0);
+    pm.assign(len, 0.0);
+    size_t q = 0, used = 0;
+    for (int i = 0; i < count; ++i) {
+      if (!nmig[i]) continue;
+      const size_t o = (size_t)(c->slots[first + i].mig_off - m0);
+      std::copy(mig_edge + q, mig_edge + q + nmig[i], pe.begin() + o);
+      std::copy(mig_to + q, mig_to + q + nmig[i], pt.begin() + o);
+      std::copy(mig_time + q, mig_time + q + nmig[i], pm.begin() + o);
+      q += nmig[i];
+      used = o + nmig[i];
+    }
+    HIPCHK(c, hipMemcpyAsync(c->d_mig_edge.p + m0, pe.data(), used * 4, hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_mig_to.p + m0, pt.data(), used * 4, hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_mig_time.p + m0, pm.data(), used * 8, hipMemcpyHostToDevice,
+                             c->stream));
+  } else if (m0 >= 0) {
+    // regions elsewhere: the events go up packed and one launch takes each
+    // slot's to its region
+    int64_t q = 0;
+    for (int i = 0; i < count; ++i) {
+      if (!nmig[i]) continue;
+      from.push_back(q);
+      to.push_back(c->slots[first + i].mig_off);
+      cnt.push_back(nmig[i]);
+      q += nmig[i];
+    }
+    const size_t m = from.size();
+    HIPCHK(c, reserve(c->d_mv_off, 2 * m));
+    HIPCHK(c, reserve(c->d_mv_cnt, m + 2 * (size_t)q));
+    HIPCHK(c, reserve(c->d_mv_time, (size_t)q));
+    int32_t *de = c->d_mv_cnt.p + m, *dt = de + q;
+    HIPCHK(c, hipMemcpyAsync(c->d_mv_off.p, from.data(), m * 8, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_mv_off.p + m, to.data(), m * 8, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_mv_cnt.p, cnt.data(), m * 4, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(de, mig_edge, (size_t)q * 4, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(dt, mig_to, (size_t)q * 4, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->d_mv_time.p, mig_time, (size_t)q * 8, hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, launch_move_events((int)m, c->d_mv_off.p, c->d_mv_off.p + m, c->d_mv_cnt.p, de, dt,
+                                 c->d_mv_time.p, c->d_mig_edge.p, c->d_mig_to.p, c->d_mig_time.p,
+                                 c->stream));
   }
   HIPCHK(c, upload_slot_meta_range(c, first, count));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -3215,7 +3142,6 @@ int ima_t_nw_update(ima_ctx *c, const int32_t *slots, int nslots, const double *
   if ((rc = upload_slot_meta(c)) != IMA_OK) return rc;
   if ((rc = upload_models(c)) != IMA_OK) return rc;
   if ((rc = nw_reserve_backups(c)) != IMA_OK) return rc;
-  if ((rc = nw_upload_slots(c, slots, nslots)) != IMA_OK) return rc;
   const int tw = P - 1;
   HIPCHK(c, reserve(c->d_pslots, nslots));
   HIPCHK(c, reserve(c->d_tv, (size_t)tw));
@@ -3263,7 +3189,7 @@ int ima_t_nw_update(ima_ctx *c, const int32_t *slots, int nslots, const double *
     if (updated) updated[i] = st[i];
     if (st[i] == 1) changed.push_back(slots[i]);
   }
-  return nw_sync_slots(c, changed.data(), (int)changed.size());
+  return sync_slot_meta(c, changed.data(), (int)changed.size());
 }
 
 int ima_treeweight(ima_ctx *c, const int32_t *slots, int nslots, const double *tvals,

@@ -44,12 +44,10 @@ struct ima_ctx {
   DevBuf<int32_t> d_mult;
   DevBuf<uint64_t> d_mask;
 
-  // genealogy slots
+  // genealogy slots: their records here and on the device, the genealogies
+  // on the device only
   std::vector<SlotMeta> slots;
   size_t nodes = 0, progs = 0;
-  std::vector<int32_t> up0, up1, down, A;
-  std::vector<double> time;
-  std::vector<ProgOp> prog;
   DevBuf<SlotMeta> d_slots;
   DevBuf<int32_t> d_up0, d_up1, d_down, d_A;
   DevBuf<double> d_time;
@@ -57,8 +55,6 @@ struct ima_ctx {
   bool slots_meta_dirty = true;
   std::vector<int> scratch_slot;  // per locus, for ima_likelihood_hky
   // population labels and migration events of the genealogies (prior)
-  std::vector<int32_t> pop, mig_edge, mig_to, mig_first, mig_count;
-  std::vector<double> mig_time;
   size_t migs = 0;
   DevBuf<int32_t> d_pop, d_mig_edge, d_mig_to, d_mig_first, d_mig_count;
   DevBuf<double> d_mig_time;
@@ -68,8 +64,11 @@ struct ima_ctx {
   DevBuf<double> d_nw_mt;
   DevBuf<int32_t> d_nw_nbk, d_nw_st, d_nw_period;
   DevBuf<double> d_nw_w, d_nw_newt;
-  DevBuf<int64_t> d_mv_off;  // event regions moved to larger ones: from | to
+  // events on their way to their regions: from | to, counts (and a write's
+  // packed edges and populations), a write's packed times
+  DevBuf<int64_t> d_mv_off;
   DevBuf<int32_t> d_mv_cnt;
+  DevBuf<double> d_mv_time;
 
   // population models of the genealogy prior
   std::vector<ModelMeta> models;

@@ -284,9 +284,11 @@ size_t nw_lds_bytes(int max_n, int max_cap, int stage);
 hipError_t launch_nw_update(const DeviceView &v, const NwArgs &a, hipStream_t st);
 hipError_t launch_nw_restore(const DeviceView &v, const NwArgs &a, const int32_t *decision,
                              hipStream_t st);
-// Copies cnt[i] events of every slot i from offset from[i] to to[i]
-// (regions that do not overlap).
+// Copies cnt[i] events of every slot i from offset from[i] of the source
+// arrays to offset to[i] of the events (regions that do not overlap, where
+// both are the same).
 hipError_t launch_move_events(int n, const int64_t *from, const int64_t *to, const int32_t *cnt,
+                              const int32_t *src_e, const int32_t *src_to, const double *src_t,
                               int32_t *me, int32_t *mto, double *mt, hipStream_t st);
 
 struct MC3Dev {

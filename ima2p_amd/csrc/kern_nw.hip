@@ -607,24 +607,27 @@ __global__ __launch_bounds__(kWave) void nw_restore_kernel(DeviceView v, NwArgs 
 
 __global__ __launch_bounds__(kWave) void move_events_kernel(int n, const int64_t *from,
                                                             const int64_t *to, const int32_t *cnt,
-                                                            int32_t *me, int32_t *mto, double *mt) {
+                                                            const int32_t *se, const int32_t *sto,
+                                                            const double *st, int32_t *me,
+                                                            int32_t *mto, double *mt) {
   const int i = blockIdx.x;
   if (i >= n) return;
   const int64_t f = from[i], t = to[i];
   for (int x = threadIdx.x; x < cnt[i]; x += kWave) {
-    me[t + x] = me[f + x];
-    mto[t + x] = mto[f + x];
-    mt[t + x] = mt[f + x];
+    me[t + x] = se[f + x];
+    mto[t + x] = sto[f + x];
+    mt[t + x] = st[f + x];
   }
 }
 
 }  // namespace
 
 hipError_t launch_move_events(int n, const int64_t *from, const int64_t *to, const int32_t *cnt,
+                              const int32_t *src_e, const int32_t *src_to, const double *src_t,
                               int32_t *me, int32_t *mto, double *mt, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(move_events_kernel, dim3(n), dim3(kWave), 0, st, n, from, to, cnt, me, mto,
-                     mt);
+  hipLaunchKernelGGL(move_events_kernel, dim3(n), dim3(kWave), 0, st, n, from, to, cnt, src_e,
+                     src_to, src_t, me, mto, mt);
   return hipGetLastError();
 }
 

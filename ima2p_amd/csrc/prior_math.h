@@ -385,8 +385,8 @@ __device__ inline double prior_param_lga(int npsize, int t, int c, const double 
 __device__ inline double prior_param_bound(const ModelView &md, int npsize, int t) {
   return t < npsize ? md.qmax[t] : md.mmax[t - npsize];
 }
-// A function of its own: inlined into the accept step it took 70 registers to
-// scratch memory and the constants of every logarithm with them.
+// A function of its own: about 900 instructions that the accept step calls
+// from two places.
 static __device__ __attribute__((noinline)) double prior_param_term_lga(int npsize, int t, int c, double f, double h,
                                               double lga, double max, double lmax) {
   return t < npsize ? pri_coalescent_term(c, f, h, max, 0.0, lga, lmax)
