@@ -240,7 +240,8 @@ size_t margincalc_work_bytes(const LTable &t, int nx);
 hipError_t upload_pow10_table(hipStream_t st);
 
 // Genealogy prior (kern_prior.hip).
-size_t treeweight_lds_bytes(int P, int emax);
+size_t treeweight_lds_bytes(int P, int emax);   // the bound on a genealogy's events
+size_t treeweight_smem_bytes(int P, int emax);  // what a launch needs
 hipError_t launch_treeweight(const DeviceView &v, const int32_t *slots, int nslots,
                              const double *tvals, const int32_t *tv_row, int P, int emax,
                              double *rec_out, int32_t *status, hipStream_t st);

@@ -561,7 +561,7 @@ hipError_t launch_hky_list(const DeviceView &v, const ima_item *items, const int
 
 size_t hky_tw_lds_bytes(int precision, int max_n, int max_slots, int ppl, int P, int emax) {
   return std::max(hky_lds_bytes(precision, max_n, max_slots, ppl),
-                  treeweight_lds_bytes(P, emax));
+                  treeweight_smem_bytes(P, emax));
 }
 
 hipError_t launch_hky_tw(const DeviceView &v, const ima_item *items, const HkyPlan &plan,

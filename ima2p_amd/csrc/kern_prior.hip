@@ -22,7 +22,7 @@ namespace {
 __global__ void __launch_bounds__(kWave)
 treeweight_kernel(DeviceView v, const int32_t *slots, int nslots, const double *tvals,
                   const int32_t *tv_row, double *rec_out, int32_t *status) {
-  extern __shared__ double lds[];
+  extern __shared__ __align__(16) double lds[];
   if ((int)blockIdx.x >= nslots) return;
   twdev::treeweight_one(v, slots, blockIdx.x, tvals, tv_row, rec_out, status, lds);
 }
@@ -61,10 +61,19 @@ prior_kernel(DeviceView v, int model, const double *recs, const int32_t *group_o
 
 }  // namespace
 
+// What limits a genealogy's events: its weights were refused beyond this, and
+// still are.
 size_t treeweight_lds_bytes(int P, int emax) {
-  // record, unsorted and sorted events, one chunk's terms
   return (size_t)prior_rec_len(P) * 8 + (size_t)emax * 24 +
          (size_t)(2 * (2 * P - 1) + 1) * kWave * 8;
+}
+
+// record and sorted events; the unsorted events and, over them, one chunk's
+// terms
+size_t treeweight_smem_bytes(int P, int emax) {
+  const size_t e4 = ((size_t)emax + 3) & ~(size_t)3, T = 2 * (size_t)P - 1;
+  return ((size_t)prior_rec_len(P) + 1) / 2 * 16 + e4 * 12 +
+         std::max(e4 * 12, (2 * T + 1) * twdev::kTermRow * 8);
 }
 
 hipError_t launch_treeweight(const DeviceView &v, const int32_t *slots, int nslots,
@@ -72,7 +81,7 @@ hipError_t launch_treeweight(const DeviceView &v, const int32_t *slots, int nslo
                              double *rec_out, int32_t *status, hipStream_t st) {
   if (nslots <= 0) return hipSuccess;
   hipLaunchKernelGGL(treeweight_kernel, dim3(nslots), dim3(kWave),
-                     treeweight_lds_bytes(P, emax), st, v, slots, nslots, tvals, tv_row,
+                     treeweight_smem_bytes(P, emax), st, v, slots, nslots, tvals, tv_row,
                      rec_out, status);
   return hipGetLastError();
 }
