@@ -68,11 +68,11 @@ size_t treeweight_lds_bytes(int P, int emax) {
          (size_t)(2 * (2 * P - 1) + 1) * kWave * 8;
 }
 
-// record and sorted events; the unsorted events and, over them, one chunk's
+// model tables, record and sorted events; the unsorted events and, over them, one chunk's
 // terms
 size_t treeweight_smem_bytes(int P, int emax) {
   const size_t e4 = ((size_t)emax + 3) & ~(size_t)3, T = 2 * (size_t)P - 1;
-  return ((size_t)prior_rec_len(P) + 1) / 2 * 16 + e4 * 12 +
+  return twdev::treeweight_tables(P) + ((size_t)prior_rec_len(P) + 1) / 2 * 16 + e4 * 12 +
          std::max(e4 * 12, (2 * T + 1) * twdev::kTermRow * 8);
 }
 

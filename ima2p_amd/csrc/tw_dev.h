@@ -30,6 +30,11 @@ enum : int { EV_COAL = 0, EV_MIG = 1, EV_SPLIT = 2 };
 // doubles from one row of terms to the next: lanes that read a row each meet
 // different banks
 constexpr int kTermRow = kWave + 2;
+// bytes of the model's tables
+__host__ __device__ constexpr size_t treeweight_tables(int P) {
+  const int T = 2 * P - 1;
+  return ((size_t)P * 8 + (size_t)(P * T + 5 * P + 2 * T) * 4 + 15) / 16 * 16;
+}
 static_assert(2 * (2 * kMaxPops - 1) + 1 <= kWave, "a lane per sum");
 
 __device__ inline int ev_pack(int type, int pop, int topop) {
@@ -57,8 +62,8 @@ __device__ inline int period_of(const double *tv, int nper, double t) {
 // sum in event order.  So the first loads of events go out with the model's,
 // the sort reads two times at once, the terms of a chunk are summed by a lane
 // each from rows in different banks, eight reads ahead of their additions,
-// and the terms lie over the unsorted events (7.0 to 5.4 KB for two
-// populations).  76800 genealogies of 30 copies on average: 210 to 149 us,
+// and the terms lie over the unsorted events (8.3 to 5.5 KB for two
+// populations).  76800 genealogies of 30 copies on average: 210 to 137 us,
 // 3200 of 45 copies and three populations 29 to 22 us.
 __device__ __forceinline__ void treeweight_one(const DeviceView &v, const int32_t *slots, int i,
                                                const double *tvals, const int32_t *tv_row,
@@ -99,11 +104,13 @@ __device__ __forceinline__ void treeweight_one(const DeviceView &v, const int32_
   }
 
   // the model's small tables, read inside the event loops, live in LDS
-  __shared__ int s_pos[kMaxPops * (2 * kMaxPops - 1)], s_join[3 * kMaxPops];
-  __shared__ int s_pope[2 * kMaxPops - 1], s_popdown[2 * kMaxPops - 1];
-  __shared__ int s_npresent[kMaxPops];
-  __shared__ double s_tv[kMaxPops];
-  __shared__ int s_spos[kMaxPops];  // sorted position of split k
+  double *s_tv = lds;                      // [P] split times
+  int *s_pos = (int *)(s_tv + P);          // [P][T]
+  int *s_join = s_pos + P * T;             // [P][3]
+  int *s_pope = s_join + 3 * P, *s_popdown = s_pope + T;  // [T]
+  int *s_npresent = s_popdown + T;         // [P]
+  int *s_spos = s_npresent + P;            // [P] sorted position of split k
+  lds += treeweight_tables(P) / 8;
   for (int x = lane; x < P * T; x += kWave) s_pos[x] = md.pos[x];
   for (int x = lane; x < 3 * P; x += kWave) s_join[x] = md.join[x];
   for (int x = lane; x < T; x += kWave) {
