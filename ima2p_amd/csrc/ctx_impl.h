@@ -91,6 +91,9 @@ struct ima_ctx {
   DevBuf<double> d_aux64;
   DevBuf<ima_sw_move> d_swmoves;  // ima_sw_update_A's moves
   DevBuf<int4> d_units, d_red;
+  // the host's lists of one scoring call
+  std::vector<int32_t> plan_idx, plan_is, plan_sw, plan_hky, plan_slots, plan_locus;
+  std::vector<int4> plan_units, plan_red;
   DevBuf<double> d_partial;
 
   // L mode
