@@ -129,6 +129,8 @@ PROTOS = {
                                           C.c_double, dp]),
     "ima_lmode_popmig": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, C.c_double, C.c_double,
                                    C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, dp, C.c_int, dp]),
+    "ima_lmode_popmig_plan": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
+                                        C.POINTER(C.c_int), C.POINTER(C.c_int64)]),
     "ima_lmode_popmig_peak": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, C.c_double, C.c_double,
                                         C.c_int, C.c_int, C.c_int, dp, dp,
                                         C.POINTER(C.c_int64)]),

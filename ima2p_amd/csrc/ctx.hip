@@ -1243,17 +1243,29 @@ int ima_lmode_popmig(ima_ctx *c, int id, int theta_i, int mig_i, double qmax, do
   if ((rc = upload_models(c)) != IMA_OK) return rc;
   const LTable t = ltable(h);
   HIPCHK(c, reserve(c->d_lx, (size_t)nx));
-  HIPCHK(c, reserve(c->d_lwork, popmig_work_bytes(t, nx) / 8 + 1));
+  const PopmigPlan plan =
+      popmig_plan(kind == IMA_POPMIG_MARGIN ? last - first : h.G, nx, expo);
+  HIPCHK(c, reserve(c->d_lwork, plan.bytes / 8 + 1));
   HIPCHK(c, reserve(c->d_lout, (size_t)nx));
   HIPCHK(c, hipMemcpyAsync(c->d_lx.p, x, (size_t)nx * 8, hipMemcpyHostToDevice, c->stream));
   if ((rc = timing_begin(c, K_LMODE)) != IMA_OK) return rc;
   HIPCHK(c, launch_popmig(t, theta_i, mig_i, qmax, mprior, expo, kind, prob_or_like, first, last,
-                          c->d_lx.p, nx, c->d_logfact.p, (int)c->logfact.size(), c->d_lwork.p,
-                          c->d_lout.p, c->stream));
+                          c->d_lx.p, nx, c->d_logfact.p, (int)c->logfact.size(), plan,
+                          c->d_lwork.p, c->d_lwork.n * 8, c->d_lout.p, c->stream));
   if ((rc = timing_end(c, K_LMODE)) != IMA_OK) return rc;
   HIPCHK(c, hipMemcpyAsync(out, c->d_lout.p, (size_t)nx * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return timing_collect(c, K_LMODE);
+}
+
+int ima_lmode_popmig_plan(int rows, int nx, int expo, int *chunks, int *chunk_rows,
+                          int64_t *work_bytes) {
+  if (!chunks || !chunk_rows || !work_bytes || rows < 1 || nx < 0) return IMA_ERR_ARG;
+  const PopmigPlan p = popmig_plan(rows, nx, expo);
+  *chunks = p.nchunks;
+  *chunk_rows = p.chunk_rows;
+  *work_bytes = (int64_t)p.bytes;
+  return IMA_OK;
 }
 
 int ima_lmode_greater_than(ima_ctx *c, int id, int kind, int n, const double *prior_max,

@@ -227,11 +227,19 @@ size_t jointp_work_bytes(const LTable &t, int npoints);
 hipError_t launch_greater_than(const LTable &t, int kind, const int2 *pairs, const double *pmax,
                                int npairs, const double *lf, int nlf, double *per, double *out,
                                hipStream_t st);
-size_t popmig_work_bytes(const LTable &t, int nx);
+// The 2NM density's split of the rows of a call (the table's, or those of
+// its range) and the work area that holds every chunk's partials.
+struct PopmigPlan {
+  bool points;  // the lanes hold points, not rows
+  int nchunks, chunk_rows;
+  size_t bytes;
+};
+PopmigPlan popmig_plan(int rows, int nx, int expo);
 hipError_t launch_popmig(const LTable &t, int theta_i, int mig_i, double qmax, double mprior,
                          int expo, int kind, int prob_or_like, int first, int last,
-                         const double *x, int nx, const double *lf, int nlf, double *work,
-                         double *out, hipStream_t st);
+                         const double *x, int nx, const double *lf, int nlf,
+                         const PopmigPlan &plan, double *work, size_t work_bytes, double *out,
+                         hipStream_t st);
 hipError_t launch_margincalc(const LTable &t, int param, const double *x,
                              int nx, int logi, double yadjust, int expo,
                              double prior_mean, double *work, double *out,

@@ -1224,16 +1224,32 @@ static void point_chunks(int G, int *nchunks, int *chunk_rows) {
   *nchunks = (G + rows - 1) / rows;
 }
 
-size_t popmig_work_bytes(const LTable &t, int nx) {
-  int nc, cr;
-  point_chunks(t.G, &nc, &cr);  // no fewer than row_chunks makes
-  return (size_t)nx * nc * 2 * sizeof(double) + 64;
+// How nx points over n rows are laid out, and the work area that takes.  The
+// chunks follow from n, the rows of the call: fewer rows than the table's
+// may make more chunks.
+//
+// A wavefront runs as long as its longest series or fraction.  Lanes that
+// hold points are at one row, and alike where many points lie close; lanes
+// that hold rows have a lone point's rows side by side.  On 20000
+// genealogies, uniform prior (exponential), in us with the call's 25: 500
+// points 621 (306) with points, 772 (723) with rows; 100 points 237 (138)
+// and 206 (180); 1 point 39 (44) with rows.
+PopmigPlan popmig_plan(int n, int nx, int expo) {
+  PopmigPlan p;
+  p.points = nx >= kRowLanes;
+  if (p.points)
+    point_chunks(n, &p.nchunks, &p.chunk_rows);
+  else
+    row_chunks(n, &p.nchunks, &p.chunk_rows);
+  p.bytes = (size_t)nx * p.nchunks * (expo ? 2 : 1) * sizeof(double);
+  return p;
 }
 
 hipError_t launch_popmig(const LTable &t, int theta_i, int mig_i, double qmax, double mprior,
                          int expo, int kind, int prob_or_like, int first, int last,
-                         const double *x, int nx, const double *lf, int nlf, double *work,
-                         double *out, hipStream_t st) {
+                         const double *x, int nx, const double *lf, int nlf,
+                         const PopmigPlan &plan, double *work, size_t work_bytes, double *out,
+                         hipStream_t st) {
   if (nx == 0) return hipSuccess;
   const JointLayout L = joint_layout(t.npsize, t.nmig);
   PArgs a{};
@@ -1260,20 +1276,17 @@ hipError_t launch_popmig(const LTable &t, int theta_i, int mig_i, double qmax, d
   a.nx = nx;
   a.lf = lf;
   a.nlf = nlf;
-  // A wavefront runs as long as its longest series or fraction.  Lanes that
-  // hold points are at one row, and alike where many points lie close; lanes
-  // that hold rows have a lone point's rows side by side.  On 20000
-  // genealogies, uniform prior (exponential), in us with the call's 25: 500
-  // points 621 (306) with points, 772 (723) with rows; 100 points 237 (138)
-  // and 206 (180); 1 point 39 (44) with rows.
-  if (nx >= kRowLanes) {
-    point_chunks(a.n, &a.nchunks, &a.chunk_rows);
+  a.nchunks = plan.nchunks;
+  a.chunk_rows = plan.chunk_rows;
+  // every row in one chunk, every partial in the work area
+  if ((int64_t)a.nchunks * a.chunk_rows < a.n ||
+      (size_t)nx * a.nchunks * (expo ? 2 : 1) * sizeof(double) > work_bytes)
+    return hipErrorInvalidValue;
+  if (plan.points)
     hipLaunchKernelGGL(popmig_points, dim3((nx + kWave - 1) / kWave, a.nchunks), dim3(kRowLanes),
                        0, st, a, work);
-  } else {
-    row_chunks(a.n, &a.nchunks, &a.chunk_rows);
+  else
     hipLaunchKernelGGL(popmig_rows, dim3(nx, a.nchunks), dim3(kRowLanes), 0, st, a, work);
-  }
   hipLaunchKernelGGL(popmig_final, dim3((nx + 3) / 4), dim3(256), 0, st, a, work, out);
   return hipGetLastError();
 }

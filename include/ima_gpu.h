@@ -296,6 +296,11 @@ int ima_lmode_marginal_peak(ima_ctx *ctx, int table_id, int param, double lower,
 int ima_lmode_popmig(ima_ctx *ctx, int table_id, int theta_i, int mig_i, double qmax,
                      double mprior, int expo, int kind, int prob_or_like, int first, int last,
                      const double *x, int nx, double *out);
+/* Host-only planning, no device needed: how ima_lmode_popmig splits nx points
+ * over `rows` genealogies (the table's, or last - first), and the device work
+ * area it takes for every chunk's partials. */
+int ima_lmode_popmig_plan(int rows, int nx, int expo, int *chunks, int *chunk_rows,
+                          int64_t *work_bytes);
 /* The peak of the 2NM density for one (theta_i, m_i) pair over genealogies
  * [first, last) (marginalopt_popmig, popmig.cpp:361-429): the
  * IMA_POPMIG_MARGIN value at 100 bins MINPARAMVAL + j upper / 100 (one

@@ -8,6 +8,11 @@ records are 177 and 326 doubles long, get smaller groups instead of larger
 launches.  The sizes are the reference's default parameter maps
 (setup_iparams, initialize.cpp:202-760) for ladder trees of 2..5
 populations.
+
+ima_lmode_popmig_plan returns the 2NM density's split of a call's rows and
+its work area: every row lies in a chunk and every partial in the area, for
+the rows of the call and not of the table (a shorter range may make more
+chunks: 16384 rows more than 16385).
 """
 import ctypes as C
 
@@ -71,3 +76,29 @@ def test_plan_rejects_bad_sizes():
     loci, lds = C.c_int(), C.c_int64()
     assert lib.ima_mc3_prior_plan(0, 1, 1, 0, 0, C.byref(loci), C.byref(lds)) == L.ERR_ARG
     assert lib.ima_mc3_prior_plan(11, 1, 1, 0, 0, C.byref(loci), C.byref(lds)) == L.ERR_ARG
+
+
+def _popmig_plan(rows, nx, expo):
+    chunks, per, work = C.c_int(), C.c_int(), C.c_int64()
+    assert L.load().ima_lmode_popmig_plan(rows, nx, expo, C.byref(chunks), C.byref(per),
+                                          C.byref(work)) == L.IMA_OK
+    return chunks.value, per.value, work.value
+
+
+@pytest.mark.parametrize("expo", [0, 1])
+@pytest.mark.parametrize("nx", [1, 255, 256, 4096])
+def test_popmig_partials_fit_their_work_area(nx, expo):
+    around = [n + d for n in (49152, 65536, 131072, 1000000, 3000000, 2 * 10 ** 9)
+              for d in (-1, 0, 1, 4097)]
+    for rows in list(range(1, 40001)) + around:
+        chunks, per, work = _popmig_plan(rows, nx, expo)
+        assert (chunks - 1) * per < rows <= chunks * per and chunks <= 1024
+        assert work >= nx * chunks * (2 if expo else 1) * 8
+
+
+def test_popmig_plan_rejects_bad_sizes():
+    a, b, w = C.c_int(), C.c_int(), C.c_int64()
+    lib = L.load()
+    assert lib.ima_lmode_popmig_plan(0, 1, 0, C.byref(a), C.byref(b), C.byref(w)) == L.ERR_ARG
+    assert lib.ima_lmode_popmig_plan(1, -1, 0, C.byref(a), C.byref(b), C.byref(w)) == L.ERR_ARG
+    assert lib.ima_lmode_popmig_plan(1, 1, 0, None, C.byref(b), C.byref(w)) == L.ERR_ARG
