@@ -1002,10 +1002,16 @@ hipError_t launch_margincalc(const LTable &t, int param, const double *x, int nx
 //     reference's special cases when the counts or sums vanish;
 //   exponential migration prior (mean mmean): its own closed form with one
 //     upper incomplete gamma.
-// For a few points the lanes hold rows, for many they hold points.  Uniform terms are summed (terms whose log lies
-// outside (-700, 700) are skipped, as the reference does); exponential-prior
-// terms are summed relative to their running maximum (log-sum-exp), the
-// reference's eexp sum to rounding.
+// For a few points the lanes hold rows, for many they hold points.  Uniform
+// terms are summed (terms whose log lies outside (-700, 700) are skipped, as
+// the reference does); exponential-prior terms are summed relative to their
+// maximum (log-sum-exp), the reference's eexp sum to rounding.
+//
+// Both layouts add the same tree, so a point's value has the same bits in any
+// batch: a chunk has 64 leaves, rows l, l + 64, ... of it, added in order; the
+// leaves are joined two by two, and the chunks as popmig_final does.  What
+// rounds is written out (no contraction: the compiler may fuse the two
+// kernels' products differently), and joining is commutative.
 
 struct PArgs {
   const float *rows;
@@ -1038,27 +1044,28 @@ __device__ inline double pm_lower(const PArgs &a, int k, double x) {
 // log of the term of one genealogy, or flags a skipped term (uniform: the
 // reference adds exp(t) only for -700 < t < 700).
 __device__ inline double popmig_term(const PArgs &a, const float *g, double x, bool *use) {
+#pragma clang fp contract(off)
   const int cc = (int)g[a.cc], mc = (int)g[a.mc];
   const double fc = g[a.fc], hc = g[a.hc], fm = g[a.fm], qintg = g[a.qi], mintg = g[a.mi];
   *use = true;
   if (!a.expo) {
     double t1, t2;
     if (fc == 0 && cc == 0 && fm > 0) {
-      t1 = kLog2 - (mc * log(fm)) - hc - qintg - mintg;
+      t1 = fma(-mc, log(fm), kLog2) - hc - qintg - mintg;
       t2 = log(exp(pm_upper(a, mc, 2 * fm * x / a.qmax)) - exp(pm_upper(a, mc, a.mmax * fm)));
     } else if (fm == 0 && mc == 0 && fc > 0) {
-      t1 = kLog2 - (cc * log(fc)) - hc - qintg - mintg;
+      t1 = fma(-cc, log(fc), kLog2) - hc - qintg - mintg;
       t2 = log(exp(pm_upper(a, cc, 2 * fc / a.qmax)) - exp(pm_upper(a, cc, fc * a.mmax / x)));
     } else if (fc == 0 && cc == 0 && mc == 0 && fm == 0) {
       t1 = log(2 * log(a.mmax * a.qmax / (2 * x))) - hc - qintg - mintg;
       t2 = 0;
     } else {
-      t1 = kLog2 + (mc * log(x)) - ((cc + mc) * log(fc + fm * x)) - hc - qintg - mintg;
-      double ua = pm_upper(a, cc + mc, 2 * (fc + fm * x) / a.qmax);
-      double ub = pm_upper(a, cc + mc, a.mmax * (fm + fc / x));
+      const double w = fma(fm, x, fc), lo = 2 * w / a.qmax, hi = a.mmax * (fm + fc / x);
+      t1 = fma(-(cc + mc), log(w), fma(mc, log(x), kLog2)) - hc - qintg - mintg;
+      double ua = pm_upper(a, cc + mc, lo), ub = pm_upper(a, cc + mc, hi);
       if (ua == ub) {  // both gammas saturate: the lower ones differ instead
-        ub = pm_lower(a, cc + mc, 2 * (fc + fm * x) / a.qmax);
-        ua = pm_lower(a, cc + mc, a.mmax * (fm + fc / x));
+        ub = pm_lower(a, cc + mc, lo);
+        ua = pm_lower(a, cc + mc, hi);
       }
       if (ua > ub) {
         t2 = pri_logdiff(ua, ub);
@@ -1071,112 +1078,114 @@ __device__ inline double popmig_term(const PArgs &a, const float *g, double x, b
     return t;
   }
   const double mmean = a.mmean;
-  const double u1 = x + fc * mmean + fm * mmean * x;
+  const double u1 = fma(fm * mmean, x, fma(fc, mmean, x));
   double t2 = kLog2 - hc - log(mmean) - qintg - mintg;
   const double t3 = 2 * u1 / (mmean * a.qmax);
   if (mc == 0 && cc == 0) {
     t2 += pm_upper(a, 0, t3);
   } else if (cc == 0) {
-    t2 += pm_upper(a, mc, t3) - mc * log(fm + 1 / mmean);
+    t2 += fma(-mc, log(fm + 1 / mmean), pm_upper(a, mc, t3));
   } else if (mc == 0) {
-    t2 += pm_upper(a, cc, t3) + -cc * log(fc + x * (fm + 1 / mmean));
+    t2 += fma(-cc, log(fma(x, fm + 1 / mmean, fc)), pm_upper(a, cc, t3));
   } else {
-    t2 += pm_upper(a, mc + cc, t3) - cc * log(x) + (cc + mc) * log(mmean * x / u1);
+    t2 = fma(cc + mc, log(mmean * x / u1), fma(-cc, log(x), t2 + pm_upper(a, mc + cc, t3)));
   }
   return t2;
 }
 
-// (m, s) and (m2, s2) as one sum relative to the larger maximum
-__device__ inline void popmig_join(double &m, double &s, double m2, double s2) {
-  if (m2 == -INFINITY && s2 == 0.0) return;  // no terms (a NaN stays)
-  const double to = fmax(m, m2);
-  s = s * exp(m - to) + s2 * exp(m2 - to);
-  m = to;
+// Terms added: s under uniform priors, s e^m under the exponential one (no
+// terms: s = 0 and m = -inf; a NaN among them is in s).
+struct PmSum {
+  double m, s;
+};
+constexpr PmSum kPmNone{-INFINITY, 0.0};
+
+__device__ inline PmSum pm_join(const PArgs &a, PmSum u, PmSum v) {
+#pragma clang fp contract(off)
+  if (!a.expo) return PmSum{u.m, u.s + v.s};
+  const bool up = v.m > u.m;
+  const PmSum hi = up ? v : u, lo = up ? u : v;
+  if (lo.m == -INFINITY && lo.s == 0.0) return hi;
+  return PmSum{hi.m, fma(lo.s, exp(lo.m - hi.m), hi.s)};
 }
 
-// row r's term at x added
-__device__ inline void popmig_add(const PArgs &a, int r, double x, double &mx, double &s) {
+// sum with row r's term at x joined
+__device__ inline PmSum pm_add(const PArgs &a, int r, double x, PmSum sum) {
   bool use;
   const double t = popmig_term(a, a.rows + (size_t)(a.g0 + r) * a.K, x, &use);
-  if (!a.expo) {
-    if (use) s += exp(t);
-  } else if (t > mx) {
-    s = s * exp(mx - t) + 1.0;
-    mx = t;
-  } else {
-    s += exp(t - mx);
-  }
+  PmSum v = kPmNone;
+  if (!a.expo)
+    v.s = use ? exp(t) : 0.0;
+  else if (t > -INFINITY)
+    v = PmSum{t, 1.0};
+  else if (t != t)
+    v.s = t;
+  return pm_join(a, sum, v);
 }
 
-// work[pt][chunk] = (sum) for uniform priors, (max, sum relative to max)
-// for the exponential prior
-__device__ inline void popmig_put(const PArgs &a, int pt, int chunk, double mx, double s,
-                                  double *work) {
+// work[pt][chunk]
+__device__ inline void popmig_put(const PArgs &a, int pt, int chunk, PmSum v, double *work) {
   const size_t o = (size_t)pt * a.nchunks + chunk;
   if (!a.expo) {
-    work[o] = s;
+    work[o] = v.s;
   } else {
-    work[2 * o] = mx;
-    work[2 * o + 1] = s;
+    work[2 * o] = v.m;
+    work[2 * o + 1] = v.s;
   }
 }
 
-// The lanes hold rows, a workgroup takes one point.
+__device__ inline bool popmig_inside(const PArgs &a, double x) {
+  return !(a.kind == IMA_POPMIG_MARGIN && (x < 0 || x > a.xmax));
+}
+
+// The lanes hold a chunk's leaves; a wavefront takes a chunk, a workgroup one
+// point.
 __global__ __launch_bounds__(kRowLanes, 4) void popmig_rows(PArgs a, double *work) {
-  __shared__ double part[kRowLanes / kWave][2];
-  const int pt = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
-  const int end = min(a.n, (chunk + 1) * a.chunk_rows);
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int pt = blockIdx.x, chunk = blockIdx.y * (kRowLanes / kWave) + wave;
+  if (chunk >= a.nchunks) return;
   const double x = a.x[pt];
-  const bool inside = !(a.kind == IMA_POPMIG_MARGIN && (x < 0 || x > a.xmax));
-  double s = 0.0, mx = -INFINITY;
-  for (int r = chunk * a.chunk_rows + tid; inside && r < end; r += kRowLanes)
-    popmig_add(a, r, x, mx, s);
-  if (!a.expo) {
-    s = lanes_sum(s);
-  } else {
-    for (int off = 32; off > 0; off >>= 1)
-      popmig_join(mx, s, __shfl_xor(mx, off, kWave), __shfl_xor(s, off, kWave));
-  }
-  if (tid % kWave == 0) {
-    part[tid / kWave][0] = s;
-    part[tid / kWave][1] = mx;
-  }
-  __syncthreads();
-  if (tid != 0) return;
-  for (int w = 1; w < kRowLanes / kWave; ++w) {
-    if (!a.expo)
-      s += part[w][0];
-    else
-      popmig_join(mx, s, part[w][1], part[w][0]);
-  }
-  popmig_put(a, pt, chunk, mx, s, work);
+  const int beg = chunk * a.chunk_rows, end = min(a.n, beg + a.chunk_rows);
+  PmSum v = kPmNone;
+  if (popmig_inside(a, x))
+    for (int r = beg + lane; r < end; r += kWave) v = pm_add(a, r, x, v);
+#pragma unroll 1
+  for (int off = 1; off < kWave; off <<= 1)
+    v = pm_join(a, v, PmSum{__shfl_xor(v.m, off, kWave), __shfl_xor(v.s, off, kWave)});
+  if (lane == 0) popmig_put(a, pt, chunk, v, work);
 }
 
-// The lanes hold points and each wavefront goes over a quarter of the chunk's
-// rows.
-__global__ __launch_bounds__(kRowLanes, 4) void popmig_points(PArgs a, double *work) {
-  __shared__ double part[kRowLanes / kWave][2][kWave];
+// The lanes hold points; a workgroup takes a chunk, each wavefront RUN of its
+// leaves.
+template <int RUN>
+__global__ __launch_bounds__(kWave / RUN *kWave, 4) void popmig_points(PArgs a, double *work) {
+  constexpr int kWaves = kWave / RUN, kTop = RUN == 16 ? 4 : 2;  // RUN = 2^kTop
+  static_assert(RUN == 1 << kTop, "whole subtrees");
+  // a lane's joined leaves that wait for others: 1, 2, 4, ... of them
+  __shared__ PmSum part[kWaves][kTop + 1][kWave];
   const int chunk = blockIdx.y, lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int pt = blockIdx.x * kWave + lane;
   const double x = a.x[min(pt, a.nx - 1)];
-  const bool inside = !(a.kind == IMA_POPMIG_MARGIN && (x < 0 || x > a.xmax));
-  const int rows = a.chunk_rows / (kRowLanes / kWave);
-  const int beg = chunk * a.chunk_rows + wave * rows, end = min(a.n, beg + rows);
-  double s = 0.0, mx = -INFINITY;
-  for (int r = beg; r < end; ++r)
-    if (inside) popmig_add(a, r, x, mx, s);
-  part[wave][0][lane] = s;
-  part[wave][1][lane] = mx;
+  const bool inside = popmig_inside(a, x);
+  const int beg = chunk * a.chunk_rows, end = min(a.n, beg + a.chunk_rows);
+#pragma unroll 1
+  for (int j = 0; j < RUN; ++j) {
+    PmSum v = kPmNone;
+    if (inside)
+      for (int r = beg + wave * RUN + j; r < end; r += kWave) v = pm_add(a, r, x, v);
+    int k = 0;  // v: 2^k leaves
+    for (; (j >> k) & 1; ++k) v = pm_join(a, part[wave][k][lane], v);
+    part[wave][k][lane] = v;
+  }
   __syncthreads();
   if (wave != 0 || pt >= a.nx) return;
-  for (int w = 1; w < kRowLanes / kWave; ++w) {
-    if (!a.expo)
-      s += part[w][0][lane];
-    else
-      popmig_join(mx, s, part[w][1][lane], part[w][0][lane]);
-  }
-  popmig_put(a, pt, chunk, mx, s, work);
+#pragma unroll 1
+  for (int step = 1; step < kWaves; step *= 2)
+    for (int w = 0; w < kWaves; w += 2 * step)
+      part[w][kTop][lane] = pm_join(a, part[w][kTop][lane], part[w + step][kTop][lane]);
+  popmig_put(a, pt, chunk, part[0][kTop][lane], work);
 }
 
 // one wavefront a point
@@ -1194,13 +1203,13 @@ __global__ __launch_bounds__(256) void popmig_final(PArgs a, const double *work,
     for (int c = lane; c < a.nchunks; c += kWave) s += work[(size_t)pt * a.nchunks + c];
     v = lanes_sum(s) / a.denom;
   } else {
-    double mx = -INFINITY, s = 0.0;
+    PmSum t = kPmNone;
     for (int c = lane; c < a.nchunks; c += kWave)
-      popmig_join(mx, s, work[2 * ((size_t)pt * a.nchunks + c)],
-                  work[2 * ((size_t)pt * a.nchunks + c) + 1]);
+      t = pm_join(a, t, PmSum{work[2 * ((size_t)pt * a.nchunks + c)],
+                              work[2 * ((size_t)pt * a.nchunks + c) + 1]});
     for (int off = 32; off > 0; off >>= 1)
-      popmig_join(mx, s, __shfl_xor(mx, off, kWave), __shfl_xor(s, off, kWave));
-    v = exp(mx + log(s) - log(a.denom));
+      t = pm_join(a, t, PmSum{__shfl_xor(t.m, off, kWave), __shfl_xor(t.s, off, kWave)});
+    v = exp(t.m + log(t.s) - log(a.denom));
   }
   if (lane != 0) return;
   if (a.kind == IMA_POPMIG_MARGIN) {
@@ -1216,31 +1225,34 @@ __global__ __launch_bounds__(256) void popmig_final(PArgs a, const double *work,
   out[pt] = v;
 }
 
-// Rows a workgroup of lanes that hold points: at most 1024 chunks, at least
-// four rows a wavefront.
-static void point_chunks(int G, int *nchunks, int *chunk_rows) {
-  const int rows = std::max(16, ((G + 1023) / 1024 + 15) / 16 * 16);
-  *chunk_rows = rows;
-  *nchunks = (G + rows - 1) / rows;
-}
-
 // How nx points over n rows are laid out, and the work area that takes.  The
-// chunks follow from n, the rows of the call: fewer rows than the table's
-// may make more chunks.
+// chunks follow from n alone, the rows of the call: whole leaves, at most
+// 1024 chunks.
 //
 // A wavefront runs as long as its longest series or fraction.  Lanes that
 // hold points are at one row, and alike where many points lie close; lanes
-// that hold rows have a lone point's rows side by side.  On 20000
-// genealogies, uniform prior (exponential), in us with the call's 25: 500
-// points 621 (306) with points, 772 (723) with rows; 100 points 237 (138)
-// and 206 (180); 1 point 39 (44) with rows.
+// that hold rows have a lone point's rows side by side, but take about 1.5 times
+// as long a term.  So points once the rows' wavefronts are more than twice
+// what the chip holds (4096) and 64 points are not mostly padding; then 16
+// leaves a wavefront where those fill the chip, else four.  Calls in us (25
+// of them copies and waiting), uniform prior:
+//   20000 rows, 1 point:     42 with rows, 118 with points (16 leaves)
+//   20000 rows, 100 points:  160, 180
+//   20000 rows, 256 points:  330, 252 (four leaves: 286)
+//   20000 rows, 500 points:  593, 399
+//   2000 rows, 256 points:   77, 117 (84)
+//   2000 rows, 500 points:   104, 116 (86)
+//   2000 rows, 2000 points:  285, 204 (229)
 PopmigPlan popmig_plan(int n, int nx, int expo) {
   PopmigPlan p;
-  p.points = nx >= kRowLanes;
-  if (p.points)
-    point_chunks(n, &p.nchunks, &p.chunk_rows);
-  else
-    row_chunks(n, &p.nchunks, &p.chunk_rows);
+  const int leaf = (n - 1) / (1024 * kWave) + 1;
+  p.chunk_rows = leaf * kWave;
+  p.nchunks = (n - 1) / p.chunk_rows + 1;
+  constexpr int64_t kFull = 4096;
+  const int64_t groups = ((int64_t)nx + kWave - 1) / kWave;
+  p.run = nx < 2 * kWave || (int64_t)nx * p.nchunks <= 2 * kFull ? 0
+          : groups * p.nchunks * 4 < kFull                       ? 4
+                                                                 : 16;
   p.bytes = (size_t)nx * p.nchunks * (expo ? 2 : 1) * sizeof(double);
   return p;
 }
@@ -1282,11 +1294,15 @@ hipError_t launch_popmig(const LTable &t, int theta_i, int mig_i, double qmax, d
   if ((int64_t)a.nchunks * a.chunk_rows < a.n ||
       (size_t)nx * a.nchunks * (expo ? 2 : 1) * sizeof(double) > work_bytes)
     return hipErrorInvalidValue;
-  if (plan.points)
-    hipLaunchKernelGGL(popmig_points, dim3((nx + kWave - 1) / kWave, a.nchunks), dim3(kRowLanes),
-                       0, st, a, work);
+  const dim3 points((nx + kWave - 1) / kWave, a.nchunks);
+  if (plan.run == 16)
+    hipLaunchKernelGGL(popmig_points<16>, points, dim3(4 * kWave), 0, st, a, work);
+  else if (plan.run == 4)
+    hipLaunchKernelGGL(popmig_points<4>, points, dim3(16 * kWave), 0, st, a, work);
   else
-    hipLaunchKernelGGL(popmig_rows, dim3(nx, a.nchunks), dim3(kRowLanes), 0, st, a, work);
+    hipLaunchKernelGGL(popmig_rows,
+                       dim3(nx, (a.nchunks + kRowLanes / kWave - 1) / (kRowLanes / kWave)),
+                       dim3(kRowLanes), 0, st, a, work);
   hipLaunchKernelGGL(popmig_final, dim3((nx + 3) / 4), dim3(256), 0, st, a, work, out);
   return hipGetLastError();
 }

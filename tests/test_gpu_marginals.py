@@ -11,6 +11,7 @@ where a workgroup takes more points or the lanes change from rows to points.
   exponential prior's changes of reference, and the rounding of a term's log
   where the compiler fuses another product in the other kernel: parts up to
   500, ten of them, 10 * 500 * 2^-53 = 6e-13.
+  A point's value must have the same bits in every batch all the same.
 * peaks and limits must equal, bit for bit, the searches run here one point
   at a time; 2NM peaks with the same number of points."""
 import numpy as np
@@ -74,6 +75,24 @@ def test_popmig_layouts_agree(engine, G, expo):
             b = np.concatenate([engine.popmig(t, 0, 1, x[i:i + 100], qmax, mpr, expo=expo, **kw)
                                 for i in range(0, nx, 100)])
             assert np.all(np.abs(a - b) <= (6e-13 + 2 * G * 2.0 ** -52) * np.abs(b))
+    engine.lmode_table_free(t)
+
+
+# one row, a chunk's edges, a few chunks, two rows a leaf; the layouts change at
+# 128 points and with the wavefronts these make
+@pytest.mark.parametrize("G", [1, 63, 65, 700, 5000, 70001])
+@pytest.mark.parametrize("expo", [False, True])
+def test_popmig_same_bits_in_any_batch(engine, G, expo):
+    rng = np.random.default_rng(G)
+    t = engine.lmode_table(_table(rng, G), NP, NM, 3)
+    qmax, mpr = 15.0, (0.8 if expo else 3.0)
+    x = rng.uniform(0.05, 10.0, 9000 if G <= 65 else 1500)
+    for kw in ({"prob_or_like": 1}, {"kind": L.POPMIG_MARGIN, "first": G // 3, "last": G}):
+        full = engine.popmig(t, 0, 1, x, qmax, mpr, expo=expo, **kw)
+        for lo, n in ((0, 1), (7, 1), (0, 63), (1, 64), (3, 65), (5, 127), (5, 128), (9, 129),
+                      (200, 255), (100, 256), (50, 700)):
+            part = engine.popmig(t, 0, 1, x[lo:lo + n], qmax, mpr, expo=expo, **kw)
+            np.testing.assert_array_equal(part, full[lo:lo + n])
     engine.lmode_table_free(t)
 
 
