@@ -1249,9 +1249,11 @@ int ima_lmode_popmig(ima_ctx *c, int id, int theta_i, int mig_i, double qmax, do
   HIPCHK(c, reserve(c->d_lout, (size_t)nx));
   HIPCHK(c, hipMemcpyAsync(c->d_lx.p, x, (size_t)nx * 8, hipMemcpyHostToDevice, c->stream));
   if ((rc = timing_begin(c, K_LMODE)) != IMA_OK) return rc;
-  HIPCHK(c, launch_popmig(t, theta_i, mig_i, qmax, mprior, expo, kind, prob_or_like, first, last,
-                          c->d_lx.p, nx, c->d_logfact.p, (int)c->logfact.size(), plan,
-                          c->d_lwork.p, c->d_lwork.n * 8, c->d_lout.p, c->stream));
+  for (int64_t p = 0; p < nx; p += plan.points)
+    HIPCHK(c, launch_popmig(t, theta_i, mig_i, qmax, mprior, expo, kind, prob_or_like, first, last,
+                            c->d_lx.p + p, (int)std::min<int64_t>(plan.points, nx - p), c->d_logfact.p,
+                            (int)c->logfact.size(), plan, c->d_lwork.p, c->d_lwork.n * 8,
+                            c->d_lout.p + p, c->stream));
   if ((rc = timing_end(c, K_LMODE)) != IMA_OK) return rc;
   HIPCHK(c, hipMemcpyAsync(out, c->d_lout.p, (size_t)nx * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -230,6 +230,7 @@ hipError_t launch_greater_than(const LTable &t, int kind, const int2 *pairs, con
 // The 2NM density's split of the rows of a call (the table's, or those of
 // its range) and the work area that holds every chunk's partials.
 struct PopmigPlan {
+  int points;  // points a launch takes
   int run;  // the lanes hold points: leaves a wavefront takes (0: they hold rows)
   int nchunks, chunk_rows;
   size_t bytes;

@@ -1227,7 +1227,8 @@ __global__ __launch_bounds__(256) void popmig_final(PArgs a, const double *work,
 
 // How nx points over n rows are laid out, and the work area that takes.  The
 // chunks follow from n alone, the rows of the call: whole leaves, at most
-// 1024 chunks.
+// 1024 chunks.  A launch takes as many points as leave the area within 64 MiB
+// (4096 or more); a call with more of them makes several.
 //
 // A wavefront runs as long as its longest series or fraction.  Lanes that
 // hold points are at one row, and alike where many points lie close; lanes
@@ -1248,12 +1249,14 @@ PopmigPlan popmig_plan(int n, int nx, int expo) {
   const int leaf = (n - 1) / (1024 * kWave) + 1;
   p.chunk_rows = leaf * kWave;
   p.nchunks = (n - 1) / p.chunk_rows + 1;
+  const size_t point = (size_t)p.nchunks * (expo ? 2 : 1) * sizeof(double);
+  nx = p.points = (int)std::min((size_t)nx, ((size_t)64 << 20) / point);
   constexpr int64_t kFull = 4096;
   const int64_t groups = ((int64_t)nx + kWave - 1) / kWave;
   p.run = nx < 2 * kWave || (int64_t)nx * p.nchunks <= 2 * kFull ? 0
           : groups * p.nchunks * 4 < kFull                       ? 4
                                                                  : 16;
-  p.bytes = (size_t)nx * p.nchunks * (expo ? 2 : 1) * sizeof(double);
+  p.bytes = nx * point;
   return p;
 }
 

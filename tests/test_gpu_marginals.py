@@ -96,6 +96,16 @@ def test_popmig_same_bits_in_any_batch(engine, G, expo):
     engine.lmode_table_free(t)
 
 
+def test_popmig_more_points_than_a_launch_takes(engine):
+    t = engine.lmode_table(_table(np.random.default_rng(8), 65536), NP, NM, 3)
+    x = np.random.default_rng(9).uniform(0.05, 10.0, 2 * 4096 + 131)  # 4096 a launch
+    full = engine.popmig(t, 0, 1, x, 15.0, 0.8, expo=True)
+    for lo in (0, 4000, 4096, 8192, len(x) - 131):
+        np.testing.assert_array_equal(engine.popmig(t, 0, 1, x[lo:lo + 131], 15.0, 0.8, expo=True),
+                                      full[lo:lo + 131])
+    engine.lmode_table_free(t)
+
+
 def _peak_one_by_one(e, t, p, lower, upper):
     def f(v):
         return e.margincalc(t, p, v)[0]

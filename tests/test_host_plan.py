@@ -96,6 +96,16 @@ def test_popmig_partials_fit_their_work_area(nx, expo):
         assert work >= nx * chunks * (2 if expo else 1) * 8
 
 
+@pytest.mark.parametrize("expo", [0, 1])
+@pytest.mark.parametrize("rows", [1, 64, 20000, 65536, 65537, 1000000, 2 * 10 ** 9])
+def test_popmig_work_area_is_bounded(rows, expo):
+    """However many points: a caller with 10^8 of them needs no more."""
+    for nx in (4096, 10 ** 5, 10 ** 8, 2 ** 31 - 1):
+        chunks, _, work = _popmig_plan(rows, nx, expo)
+        per = chunks * (2 if expo else 1) * 8
+        assert min(nx, 4096) * per <= work <= 64 << 20
+
+
 def test_popmig_plan_rejects_bad_sizes():
     a, b, w = C.c_int(), C.c_int(), C.c_int64()
     lib = L.load()
