@@ -9,6 +9,10 @@ the logarithms of at most 1e5 in size that make an integral are within 2 ulp,
 so the values agree to 1e-15 of the largest of them; the tolerance is the
 path's own 1e-10 relative, with 1e-9 absolute for values near zero.
 
+Logarithm: a migration rate without events and with weight f far above 1 /
+its bound integrates to -log f exactly as the device takes the logarithm,
+which must lie within an ulp of it.
+
 Decisions: for 2 to 5 populations (up to 326 weight entries, 44 parameters)
 group sizes give the same sweeps bit for bit, and probg is the oracle's.
 """
@@ -57,6 +61,28 @@ def test_integrals(engine, qmax, mmax):
     for x in range(n):
         np.testing.assert_allclose(q[x], want[x][1], rtol=1e-10, atol=1e-9, err_msg=str(rec[x]))
         np.testing.assert_allclose(m[x], want[x][2], rtol=1e-10, atol=1e-9, err_msg=str(rec[x]))
+
+
+def test_logarithm_within_an_ulp(engine):
+    pt, theta, ts, mig = sim.im_model_two_pop()
+    model = immodel.build(pt, qmax=20.0, mmax=1e8)  # f mmax > 710: e^(-f mmax) drops out
+    mid = engine.model_add(model)
+    rng = np.random.default_rng(5)
+    f = np.concatenate([rng.uniform(0.5, 2.0, 60000), np.exp(rng.uniform(-11.0, 40.0, 20000)),
+                        1.0 + np.ldexp(rng.uniform(-1.0, 1.0, 20000), -rng.integers(1, 50, 20000))])
+    rec = np.zeros((len(f), 3 * 4 + 2 * 8 + 1))
+    k, i, j = model.mig_wp[0][0]
+    rec[:, 20 + (k * 2 + i) * 2 + j] = f
+    n = len(rec)
+    q, m, pg = np.zeros((n, model.npsize)), np.zeros((n, model.nmig)), np.zeros(n)
+    dp = lambda a: a.ctypes.data_as(L.dp)  # noqa: E731
+    for lo in range(0, n, 1000):
+        r = np.ascontiguousarray(rec[lo:lo + 1000])
+        engine._chk(engine.lib.ima_integrate_tree_prob(
+            engine.h, mid, dp(r), len(r), dp(pg[lo:]), dp(q[lo:]), dp(m[lo:])),
+            "integrate_tree_prob")
+    want = -np.log(f.astype(np.longdouble))
+    assert np.all(np.abs(m[:, 0] - want) <= np.spacing(np.abs(want).astype(np.float64)))
 
 
 def _chains(P, C_, Lc, seed):
