@@ -18,10 +18,14 @@
 // parameter's integral for 63 scenarios, three wavefronts a SIMD: about 450
 // dependent FP64 instructions with the library's logarithm (60, 3 to 5 uses),
 // exponential (40) and division (15, two a term of the fraction), 2.4 to 4.5
-// us.  So: logarithm, exponential and division below in 30, 20 and 8
+// us.  So: logarithm, exponential and division below in 32, 24 and 8
 // instructions, the fraction and the series as numerator and denominator
-// recurrences with one division at the end, and log x from the log of the
-// weight it is made of: 2.2 to 3.4 us.
+// recurrences with one division at the end, and the logarithms of the weight
+// and of the gamma's argument side by side.  The argument's could be pieced
+// together from the weight's and the bound's, and the logarithm take five
+// instructions less: 2.2 to 3.4 us, and 107 us for the accept launch of 64
+// chains x 50 loci instead of 110, but two coalescences over [0, 20] then
+// integrate with 0.52 ulp root mean square instead of 0.44.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -48,10 +52,10 @@ __device__ __forceinline__ double pri_div(double n, double d) {
 // (2 + f): log m = 2 atanh(s) = f - (f^2/2 - s (f^2/2 + R)), R = 2 (atanh(s) /
 // s - 1) by a polynomial in s^2 (interpolation of atanh(s) / s at Chebyshev
 // nodes, 5e-18 relative), so that what is rounded is small beside f; e ln 2 +
-// f is added as a sum and its rest.  Within 0.84 ulp of the logarithm, 0.295
-// root mean square (an exact one, rounded: 0.289; 2 atanh(s) itself, rounded
-// in s: 1.98 and 0.46).  No branches and no call of the library: at the integrals' many uses either
-// would fill the instruction cache.
+// f is added as a sum and its rest.  Within 0.87 ulp of the logarithm, 0.295
+// root mean square (the library's: 0.293; 2 atanh(s) itself, rounded in s:
+// 1.98 and 0.46).  No branches and no call of the library: at the integrals'
+// many uses either would fill the instruction cache.
 __device__ __forceinline__ double pri_log(double x) {
 #pragma clang fp contract(off)
   double m = __builtin_amdgcn_frexp_mant(x);
@@ -59,19 +63,22 @@ __device__ __forceinline__ double pri_log(double x) {
   const bool lo = m < 0.70710678118654752440;
   m = lo ? m + m : m;
   e = lo ? e - 1 : e;
-  const double f = m - 1.0, s = pri_div(f, 2.0 + f), z = s * s;
-  double p = 0.07308224842521703;
-  p = fma(p, z, 0.07665860800278021);
-  p = fma(p, z, 0.09091444562630861);
-  p = fma(p, z, 0.1111110556739754);
-  p = fma(p, z, 0.14285714312987743);
-  p = fma(p, z, 0.19999999999949752);
-  p = fma(p, z, 0.3333333333333335);
+  const double f = m - 1.0, d = 2.0 + f, h = 0.5 * f * f;
+  double q = __builtin_amdgcn_rcp(d);
+  q = fma(fma(-d, q, 1.0), q, q);
+  q = fma(fma(-d, q, 1.0), q, q);
+  const double s = f * q, z = s * s;
+  double p = 0.14616449685043406;
+  p = fma(p, z, 0.15331721600556042);
+  p = fma(p, z, 0.1818288912526122);
+  p = fma(p, z, 0.2222221113479488);
+  p = fma(p, z, 0.28571428625986754);
+  p = fma(p, z, 0.39999999999899504);
+  p = fma(p, z, 0.666666666666667);
   // ln 2 in two parts, the first of 32 bits: e times it is exact
-  const double k = e, h = 0.5 * f * f;
-  const double u = h - fma(s, fma(z + z, p, h), k * 1.90821492927058770002e-10);
-  const double kl = k * 6.93147180369123816490e-01, a = kl + f, b = (kl - a) + f;
-  const double r = a + (b - u);
+  const double k = e, a = fma(k, 6.93147180369123816490e-01, f);
+  const double b = fma(k, 6.93147180369123816490e-01, -a) + f;
+  const double r = a + (fma(s, fma(z, p, h), fma(k, 1.90821492927058770002e-10, b)) - h);
   // 0, infinity, negative numbers and NaN
   const double odd = x == 0.0 ? -INFINITY : x > 0.0 ? x : NAN;
   return x > 0.0 && x < INFINITY ? r : odd;
@@ -79,8 +86,9 @@ __device__ __forceinline__ double pri_log(double x) {
 
 // e^x = 2^n e^r, r = x - n ln 2 through the two parts of ln 2 with the
 // rounding of the second kept, 1 + r added as a sum and its rest: within 0.75
-// ulp (0.93 with r rounded once and 1 + r p(r) for the end).  0 and infinity
-// beyond the range come from the scaling, NaN passes through.
+// ulp, 0.293 root mean square (the library's: 0.86 and 0.302; r rounded once
+// and 1 + r p(r) for the end: 0.93 and 0.304).  0 and infinity beyond the
+// range come from the scaling, NaN passes through.
 __device__ __forceinline__ double pri_exp(double x) {
 #pragma clang fp contract(off)
   x = x > 1e5 ? 1e5 : x < -1e5 ? -1e5 : x;
@@ -276,8 +284,8 @@ __device__ inline double pri_coalescent_term(int cc, double fc, double hcc, doub
       // cc = 1: order 0, the exponential integral; else one series serves
       // both gammas
       GammaPrep gp{};
-      const double lfc = pri_log(fc);
-      if (cc > 1) gp = pri_gamma_prep(cc - 1, 2 * fc / max, lfc + (kLog2 - lmax), lga);
+      const double x = 2 * fc / max, lfc = pri_log(fc), lx = pri_log(x);
+      if (cc > 1) gp = pri_gamma_prep(cc - 1, x, lx, lga);
       double ug = cc > 1 ? pri_upper_of(gp) : pri_uppergamma(0, 2 * fc / max, lga);
       if (cc > 1) {
         const double fullg = lga;
@@ -313,15 +321,15 @@ __device__ inline double pri_coalescent_term(int cc, double fc, double hcc, doub
   return p;
 }
 
-// log int_min^max m^cm e^(-fm m) dm; lga = log(cm!), lmax = log max
+// log int_min^max m^cm e^(-fm m) dm; lga = log(cm!)
 __device__ inline double pri_migration_term(int cm, double fm, double max, double min,
-                                            double lga, double lmax) {
+                                            double lga) {
   const double mpriormin = 0.000001;  // MPRIORMIN, imamp.hpp:141
   double p;
   if (cm > 0) {
     if (min == 0) {
-      const double lfm = pri_log(fm);
-      const GammaPrep gp = pri_gamma_prep(cm + 1, fm * max, lfm + lmax, lga);
+      const double lfm = pri_log(fm), lx = pri_log(fm * max);
+      const GammaPrep gp = pri_gamma_prep(cm + 1, fm * max, lx, lga);
       double lg = pri_lower_of(gp);
       const double fullg = lga;
       if (fullg - lg < 1e-15 || fullg - lg > 7.0978271289338397e+02) {
@@ -399,7 +407,7 @@ __device__ inline double prior_param_bound(const ModelView &md, int npsize, int 
 static __device__ __attribute__((noinline)) double prior_param_term_lga(int npsize, int t, int c, double f, double h,
                                               double lga, double max, double lmax) {
   return t < npsize ? pri_coalescent_term(c, f, h, max, 0.0, lga, lmax)
-                    : pri_migration_term(c, f, max, 0.0, lga, lmax);
+                    : pri_migration_term(c, f, max, 0.0, lga);
 }
 
 __device__ inline double prior_param_term(const ModelView &md, int npsize, int t, int c,

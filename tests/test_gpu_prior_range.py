@@ -13,6 +13,12 @@ Logarithm: a migration rate without events and with weight f far above 1 /
 its bound integrates to -log f exactly as the device takes the logarithm,
 which must lie within an ulp of it.
 
+Two coalescences of weight f over [0, max], 2 f / max >= 2: the fraction ends
+at its first term, and the integral is log 2 - log f - 2 f / max, through the
+logarithms of f and of the gamma's argument.  Rounding as written with an
+exact logarithm gives 0.443 ulp root mean square at max = 20, the argument's
+logarithm pieced together from others 0.515.
+
 Decisions: for 2 to 5 populations (up to 326 weight entries, 44 parameters)
 group sizes give the same sweeps bit for bit, and probg is the oracle's.
 """
@@ -83,6 +89,26 @@ def test_logarithm_within_an_ulp(engine):
             "integrate_tree_prob")
     want = -np.log(f.astype(np.longdouble))
     assert np.all(np.abs(m[:, 0] - want) <= np.spacing(np.abs(want).astype(np.float64)))
+
+
+def test_two_coalescences_round_as_written(engine):
+    pt, theta, ts, mig = sim.im_model_two_pop()
+    model = immodel.build(pt, qmax=20.0, mmax=5.0)
+    mid = engine.model_add(model)
+    f = np.random.default_rng(6).uniform(20.0, 60.0, 40000)
+    rec = np.zeros((len(f), 3 * 4 + 2 * 8 + 1))
+    k, i = model.theta_wp[0][0]
+    rec[:, k * 2 + i] = 2
+    rec[:, 4 + k * 2 + i] = f
+    n = len(rec)
+    q, m, pg = np.zeros((n, model.npsize)), np.zeros((n, model.nmig)), np.zeros(n)
+    dp = lambda a: a.ctypes.data_as(L.dp)  # noqa: E731
+    engine._chk(engine.lib.ima_integrate_tree_prob(engine.h, mid, dp(rec), n, dp(pg), dp(q), dp(m)),
+                "integrate_tree_prob")
+    F = f.astype(np.longdouble)
+    want = np.log(np.longdouble(2)) - np.log(F) - 2 * F / 20
+    off = ((q[:, 0] - want) / np.spacing(np.abs(want).astype(np.float64))).astype(np.float64)
+    assert np.sqrt((off ** 2).mean()) <= 1.05 * 0.443
 
 
 def _chains(P, C_, Lc, seed):
