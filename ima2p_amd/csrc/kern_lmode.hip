@@ -63,9 +63,11 @@ constexpr int kXLanes = 256;
 // fused multiply-adds and the summation order (about 1e-16 relative).  A
 // batch of points against a table is therefore a matrix product, genealogies
 // x (1 + 2 parameters) x points, followed by an exp and a sum over the
-// genealogies.  It runs on the FP64 matrix unit, in logarithms to base 2
-// (the points' coefficients carry log2 e), so a term is 2^(p - M) without a
-// split-constant reduction.
+// genealogies.  It runs on the FP64 matrix unit.  (In logarithms to base 2 a
+// term's exponential takes one operation less, 4.01 ms for the surface below
+// instead of 4.15, but the base terms and coefficients are then rounded once
+// more, the result is 1.1 to 1.4 times as far from 64 bits, and terms overflow
+// from 1.25e308 on.)
 //
 // One workgroup of four wavefronts takes one chunk of rows and up to
 // 16 * T points.  It stages kRows rows at a time in LDS as FP64 records
@@ -78,22 +80,25 @@ constexpr int kXLanes = 256;
 // the table and the parameter range alone: a point's value is the same
 // alone and batched with others.
 //
-// Bound: FP64 issue, 18 vector operations per (point, genealogy) pair
-// (subtract, round, 11 multiply-adds, ldexp, the maximum and two sums; 2.2 ns
-// per 64 lanes) and the product (48 ns per 16 x 16 x 4 on a SIMD).  The two
+// Bound: FP64 issue, 20 vector operations per (point, genealogy) pair
+// (subtract, scale, round, 12 multiply-adds, conversion and ldexp, the maximum
+// and two sums; 2.2 ns per 64 lanes) and the product (48 ns per 16 x 16 x 4 on a SIMD).  The two
 // share their issue here: a loop of half of each takes the sum of both.
 // Multiply-adds in place of the product would cost 22 ns instead of 36 per
 // 64 pairs at five parameters, but the row values then pass through LDS once
-// per lane: 4.5 ms where this takes 3.9 (4096 points on 1e6 genealogies).
+// per lane: 4.5 ms where this took 3.9 (4096 points on 1e6 genealogies).
 // With one lane per point (rows in order, the library's exp and a branch on
 // every new maximum) that surface took 6.45 ms, 500 points on 1e5 in
 // REF_COMPAT 277 us, and one point on 1e5 171 us (one lane of 256 working);
-// here 4.0 ms, 111 us and 13 us.
+// here 4.15 ms, 111 us and 13 us.
 typedef double dvec4 __attribute__((ext_vector_type(4)));
 
 constexpr double kLog2E = 1.4426950408889634074;
-constexpr double kBadCoef = 1e250;  // |count or weight| <= 3.4e38: no overflow below it
-constexpr double kPadRow = -1e300;  // c0 of the rows past the end: 2^(p - M) = 0
+constexpr double kLn10 = 2.3025850929940456840;
+// Coefficients, and counts and weights (a row's base term: their product),
+// beyond this take the careful path: below it a term's size is under 1e24.
+constexpr double kBadSize = 1e11;
+constexpr double kPadRow = -1e25;  // c0 of the rows past the end: e^(p - M) = 0
 
 template <int NR>
 struct XShape {
@@ -113,34 +118,32 @@ struct XShape {
   static constexpr int kEnd = (kAdd ? 0 : 1) + 2 * NR;
 };
 
-// 2^(f + n), f in [-1/2, 1/2], exactly 2^n at f = 0: a polynomial of degree
-// 11 (interpolation at the Chebyshev nodes, 2e-17 relative), scaled.
-__device__ __forceinline__ double exp2_scaled(double f, int n) {
-  double p = 4.4558179083360645e-10;
-  p = fma(p, f, 7.074194297288521e-09);
-  p = fma(p, f, 1.0178057087733941e-07);
-  p = fma(p, f, 1.3215432535912375e-06);
-  p = fma(p, f, 1.5252733841556773e-05);
-  p = fma(p, f, 0.00015403530463724353);
-  p = fma(p, f, 0.001333355814640647);
-  p = fma(p, f, 0.009618129107587256);
-  p = fma(p, f, 0.055504108664821625);
-  p = fma(p, f, 0.24022650695910158);
-  p = fma(p, f, 0.6931471805599453);
-  p = fma(p, f, 1.0);
-  return ldexp(p, n);
+// e^t, |t| < 1e26 and e^t in range: 2^n e^r with r = t - n ln 2, |r| <= ln 2 /
+// 2, by a polynomial of degree 11 (interpolation at the Chebyshev nodes, 2e-17
+// relative), exactly 1 at t = 0.  ln 2 is one constant: r is off by n 2.3e-17,
+// which counts for terms near the largest only, where n is small.  Far below
+// the range r is anything to 1e10, and the scaling gives 0 all the same.
+__device__ __forceinline__ double exp_fast(double t) {
+  const double n = rint(t * kLog2E), r = fma(-n, kLn2, t);
+  double p = 2.5110037605963777e-08;
+  p = fma(p, r, 2.763263963904103e-07);
+  p = fma(p, r, 2.755724091857897e-06);
+  p = fma(p, r, 2.4801485482328494e-05);
+  p = fma(p, r, 0.00019841269890047113);
+  p = fma(p, r, 0.0013888888952314775);
+  p = fma(p, r, 0.008333333333319601);
+  p = fma(p, r, 0.0416666666664881);
+  p = fma(p, r, 0.1666666666666668);
+  p = fma(p, r, 0.5000000000000019);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return ldexp(p, (int)n);
 }
-// 2^t; the conversion to int saturates, so any finite t below the range
-// gives 0
-__device__ __forceinline__ double exp2_fast(double t) {
-  const double n = rint(t);
-  return exp2_scaled(t - n, (int)n);
-}
-// 2^t for any t <= 0, infinite or NaN too
-__device__ __forceinline__ double exp2_any(double t) { return t < -1100.0 ? 0.0 : exp2_fast(t); }
+// e^t for any t <= 0, infinite or NaN too
+__device__ __forceinline__ double exp_any(double t) { return t < -800.0 ? 0.0 : exp_fast(t); }
 
 // Rows [g0, g0 + cnt) as records in sh, rows cnt .. kRows - 1 as padding.
-// Returns whether this thread met a value that is not finite.
+// Returns whether this thread met a value that is not finite, or large.
 template <int NR>
 __device__ inline bool stage_rows(const LArgs &a, double *sh, int g0, int cnt) {
   using X = XShape<NR>;
@@ -181,12 +184,12 @@ __device__ inline bool stage_rows(const LArgs &a, double *sh, int g0, int cnt) {
       }
       o[X::at(k)] = c;
       o[X::at(k) + 1] = w;
-      bad = bad || !isfinite(c) || !isfinite(w);
+      bad = bad || !(fabs(c) < kBadSize) || !(fabs(w) < kBadSize);
     }
-    bad = bad || !isfinite(base);
+    bad = bad || !(fabs(base) < kBadSize * kBadSize);
 #pragma unroll
     for (int k = X::kEnd; k < X::kKP; ++k) o[k] = 0.0;
-    *c0 = base * kLog2E;
+    *c0 = base;
   }
   return bad;
 }
@@ -211,9 +214,7 @@ __device__ inline void stage_points(const LArgs &a, double *sh, int *ptbad, int 
       A = log(v);
       F = -v;
     }
-    A *= kLog2E;
-    F *= kLog2E;
-    if (!(fabs(A) < kBadCoef) || !(fabs(F) < kBadCoef)) ptbad[p] = 1;
+    if (!(fabs(A) < kBadSize) || !(fabs(F) < kBadSize)) ptbad[p] = 1;
     double *o = sh + ((size_t)(p / 16) * X::kKP) * 16 + p % 16;
     o[X::at(k) * 16] = A;
     o[(X::at(k) + 1) * 16] = F;
@@ -259,7 +260,7 @@ struct PointFrag {
   }
 };
 
-// log2 terms of the lane's point for rows 4 (lane / 16) + i of row tile t
+// terms (logs) of the lane's point for rows 4 (lane / 16) + i of row tile t
 template <int NR>
 __device__ __forceinline__ void terms(const RowFrag<NR> &a, const PointFrag<NR> &b,
                                       dvec4 (&p)[XShape<NR>::kRT]) {
@@ -311,14 +312,14 @@ __device__ __forceinline__ XPlace x_place(const LArgs &a) {
 }
 
 // --------------------------------------------------------------- EXACT --
-// Per (point, chunk): a reference M (base 2) and s = sum 2^(p - M), s2 = sum
-// 2^(2(p - M)) for the effective sample number.  M is a value the lane met
-// and at most 2^kSlack below its largest: FP64's range takes the difference,
+// Per (point, chunk): a reference M and s = sum e^(p - M), s2 = sum
+// e^(2(p - M)) for the effective sample number.  M is a value the lane met
+// and at most kSlack below its largest: FP64's range takes the difference,
 // so sums are rescaled when a term leaves it, not on every new maximum.
 struct XPart {
   double M, s, s2;
 };
-constexpr double kSlack = 200.0;
+constexpr double kSlack = 50.0;
 
 template <int NR, int T>
 __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work) {
@@ -338,10 +339,14 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
     M[j] = -DBL_MAX;
     s[j] = s2[j] = 0.0;
   }
+  // rbad: the careful path from the first stage with such a row on, so that
+  // padding (behind the last row) is only added to references above it
+  bool rbad = false;
   for (int g0 = w.gbeg; g0 < w.gend; g0 += X::kRows) {
     const int cnt = min(X::kRows, w.gend - g0);
     __syncthreads();
-    const bool rbad = __syncthreads_or(stage_rows<NR>(a, sh, g0, cnt)) != 0;
+    const bool bad = stage_rows<NR>(a, sh, g0, cnt);
+    rbad = __syncthreads_or(bad || rbad) != 0;
     if (w.wave * (X::kRows / 4) >= cnt) continue;  // only padding in this quarter
     RowFrag<NR> r;
     r.load(sh, w.wave, w.lane);
@@ -356,7 +361,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
           if (w.row0 + x / 4 * 16 + x % 4 >= cnt) continue;
           const double v = pick<NR>(p, x);
           const bool up = v > M[j];
-          const double e = exp2_any(up ? M[j] - v : v - M[j]);
+          const double e = exp_any(up ? M[j] - v : v - M[j]);
           s[j] = up ? s[j] * e + 1.0 : s[j] + e;
           s2[j] = up ? s2[j] * e * e + 1.0 : fma(e, e, s2[j]);
           M[j] = up ? v : M[j];
@@ -367,7 +372,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
       if (__any(m - M[j] > kSlack)) {
         // the reference moves up to the largest of these (the first rows'
         // way in, too: M is below everything)
-        const double to = m - M[j] > kSlack ? m : M[j], sc = exp2_fast(M[j] - to);
+        const double to = m - M[j] > kSlack ? m : M[j], sc = exp_any(M[j] - to);
         s[j] *= sc;
         s2[j] *= sc * sc;
         M[j] = to;
@@ -376,7 +381,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
       for (int t = 0; t < X::kRT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const double e = exp2_fast(p[t][i] - M[j]);
+          const double e = exp_fast(p[t][i] - M[j]);
           s[j] += e;
           s2[j] = fma(e, e, s2[j]);
         }
@@ -387,8 +392,11 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
   __syncthreads();
   XPart *part = reinterpret_cast<XPart *>(sh);
 #pragma unroll
-  for (int j = 0; j < T; ++j)
-    part[w.part * (T * 16) + j * 16 + (w.lane & 15)] = XPart{M[j], s[j], s2[j]};
+  for (int j = 0; j < T; ++j) {
+    const bool none = !rbad && !pbad[j] && M[j] < 0.1 * kPadRow;  // padding alone
+    part[w.part * (T * 16) + j * 16 + (w.lane & 15)] =
+        none ? XPart{-DBL_MAX, 0.0, 0.0} : XPart{M[j], s[j], s2[j]};
+  }
   __syncthreads();
   const int pt = w.pt0 + (int)threadIdx.x;
   if (threadIdx.x < T * 16 && pt < a.npoints) {
@@ -399,7 +407,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
     for (int k = 0; k < 16; ++k) {
       const XPart q = part[k * (T * 16) + threadIdx.x];
       if (q.s == 0.0) continue;
-      const double sc = exp2_any(q.M - o.M);
+      const double sc = exp_any(q.M - o.M);
       o.s += q.s * sc;
       o.s2 += q.s2 * sc * sc;
     }
@@ -431,14 +439,14 @@ __global__ __launch_bounds__(256) void jointp_exact_final(LArgs a, const XPart *
   double s = 0.0, s2 = 0.0;
   for (int c = lane; c < a.nchunks; c += kWave) {
     if (w[c].s == 0.0) continue;
-    const double sc = exp2_any(w[c].M - M);
+    const double sc = exp_any(w[c].M - M);
     s += w[c].s * sc;
     s2 += w[c].s2 * sc * sc;
   }
   s = wave_add(s);
   s2 = wave_add(s2);
   if (lane == 0) {
-    out[pt] = log((double)a.G) - (M * kLn2 + log(s));
+    out[pt] = log((double)a.G) - (M + log(s));
     if (ess) ess[pt] = s * s / s2;
   }
 }
@@ -457,13 +465,12 @@ __global__ __launch_bounds__(256) void jointp_exact_final(LArgs a, const XPart *
 // lies outside the window; final: the chunks merged and the list cap.
 //
 // A kept value's term is e^p / 10^maxz (the mantissa m 10^(z - maxz) of the
-// reference's eexp, utilities.cpp:1507-1539), taken here as 2^(p - maxz log2 10): the window, the list
-// cap and the ordering of the running maximum are the reference's, the term
+// reference's eexp, utilities.cpp:1507-1539), taken here as exp(p - maxz ln
+// 10): the window, the list cap and the ordering of the running maximum are the reference's, the term
 // itself differs from the degree-10 Taylor series of eexp by at most its
 // truncation, ~4e-10 relative, which moves the result by less than 1e-12
 // relative.
-constexpr double kWindow2 = 10.0 * kLog2E;
-constexpr double kLog2Of10 = 3.3219280948873623479;
+constexpr double kWindow = 10.0;
 
 // Per (point, chunk) record of pass 2: sums of the window's terms and of
 // their squares, its smallest value, its size, and whether a kept value
@@ -474,8 +481,8 @@ struct RefPart {
 };
 
 // maxz: eexp's exponent of the largest term (10^z <= e^p < 10^(z + 1)) less 10
-__device__ inline int ref_maxz(double Mfin2) {
-  return (int)floor(Mfin2 * 0.30102999566398119521) - 10;
+__device__ inline int ref_maxz(double Mfin) {
+  return (int)floor(Mfin * 0.43429448190325182765) - 10;
 }
 
 template <int NR, int T>
@@ -528,7 +535,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_max(LArgs a, double *cm
   }
 }
 
-// The log2 term of one point (its parameters x) for one table row.
+// The term (log) of one point (its parameters x) for one table row.
 __device__ inline double one_term(const LArgs &a, const float *g, const double *x) {
   const JointLayout L = joint_layout(a.npsize, a.nmig);
   double p;
@@ -550,7 +557,7 @@ __device__ inline double one_term(const LArgs &a, const float *g, const double *
       p += (double)g[L.mcp + i - a.npsize] * log(x[i]) - (double)g[L.fmp + i - a.npsize] * x[i];
     }
   }
-  return p * kLog2E;
+  return p;
 }
 
 // Per point, cmax[c] becomes the maximum over the chunks before c, and mfin
@@ -576,7 +583,7 @@ __global__ __launch_bounds__(256) void jointp_ref_prefix(LArgs a, double *cmax, 
     before = fmax(before, __shfl(v, kWave - 1, kWave));
   }
   if (lane == 0) mfin[pt] = before;
-  if (before - first >= kWindow2 + 1.0)  // clear of rounding: the kernel takes its own first value
+  if (before - first >= kWindow + 1.0)  // clear of rounding: the kernel takes its own first value
     for (int c = lane; c < a.nchunks; c += kWave) cm[c] = before;
 }
 
@@ -600,7 +607,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
     const int pt = min(w.pt0 + j * 16 + (w.lane & 15), a.npoints - 1);
     run[j] = before[(size_t)pt * a.nchunks + w.chunk];
     Mf[j] = mfin[pt];
-    sc[j] = (double)ref_maxz(Mf[j]) * kLog2Of10;
+    sc[j] = (double)ref_maxz(Mf[j]) * kLn10;
     seen[j] = -DBL_MAX;
     o[j] = RefPart{0.0, 0.0, DBL_MAX, 0, 0};
     open = open || run[j] < Mf[j];
@@ -620,7 +627,7 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
     for (int j = 0; j < T; ++j) {
       dvec4 p[X::kRT];
       terms<NR>(r, b[j], p);
-      if (g0 == 0 && w.part == 0 && !(Mf[j] - p[0][0] < kWindow2)) o[j].outside = 1;
+      if (g0 == 0 && w.part == 0 && !(Mf[j] - p[0][0] < kWindow)) o[j].outside = 1;
       if (look) {
         // candidates: within the window of the maximum before the chunk
         bool cand = false;
@@ -628,8 +635,8 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
         for (int t = 0; t < X::kRT; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            cand = cand || (w.row0 + t * 16 + i < cnt && run[j] - p[t][i] < kWindow2 &&
-                            !(Mf[j] - p[t][i] < kWindow2));
+            cand = cand || (w.row0 + t * 16 + i < cnt && run[j] - p[t][i] < kWindow &&
+                            !(Mf[j] - p[t][i] < kWindow));
         if (__syncthreads_or(cand && !o[j].outside)) {
           // with the running maximum before each value: the earlier chunks
           // (run), the earlier stages (seen), the earlier wavefronts of this
@@ -666,8 +673,8 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
             for (int i = 0; i < 4; ++i) {
               if (row + i >= cnt) continue;
               const double v = pick<NR>(p, 4 * t + i);
-              const bool kept = st - v < kWindow2;
-              if (kept && !(Mf[j] - v < kWindow2)) o[j].outside = 1;
+              const bool kept = st - v < kWindow;
+              if (kept && !(Mf[j] - v < kWindow)) o[j].outside = 1;
               if (kept && v > st) st = v;
             }
           }
@@ -684,12 +691,12 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
       for (int t = 0; t < X::kRT; ++t) {
         const int row = w.row0 + t * 16;
         const double lo = Mf[j] - fmax(fmax(p[t][0], p[t][1]), fmax(p[t][2], p[t][3]));
-        if (!__any(lo < kWindow2)) continue;
+        if (!__any(lo < kWindow)) continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const double v = p[t][i];
-          const bool in = row + i < cnt && Mf[j] - v < kWindow2;
-          const double e = in ? exp2_fast(v - sc[j]) : 0.0;
+          const bool in = row + i < cnt && Mf[j] - v < kWindow;
+          const double e = in ? exp_fast(v - sc[j]) : 0.0;
           o[j].sum += e;
           o[j].sum2 = fma(e, e, o[j].sum2);
           o[j].cnt += in ? 1 : 0;
@@ -747,11 +754,11 @@ __global__ __launch_bounds__(256) void jointp_ref_final(LArgs a, const double *m
   }
   if (lane != 0) return;
   if (!outside && cnt > 1) {  // the list cap drops the smallest kept value
-    const double e = exp2_fast(minp - (double)maxz * kLog2Of10);
+    const double e = exp_fast(minp - maxz * kLn10);
     sum -= e;
     sum2 -= e * e;
   }
-  out[pt] = log((double)a.G) - (log(sum) + maxz * 2.3025850929940456840);
+  out[pt] = log((double)a.G) - (log(sum) + maxz * kLn10);
   if (ess) ess[pt] = sum * sum / sum2;
 }
 

@@ -9,6 +9,11 @@ products below 2^12 in size, so its rounding is below 33 * 2^12 * 2^-53 =
 terms come from eexp's degree-10 Taylor series on [0, ln 2), which falls
 short by up to (ln 2)^11 / 11! = 4.5e-10 of a term (REF_TOL); the engine's
 do not.  The same points are the same bits alone and in any batch.
+
+Rounding: against 80-bit values REF_COMPAT's error over a table's points (2-norm
+over that of the values, root mean square over tables of all sizes of terms) is
+2.2e-16 with terms, coefficients and exponentials rounded once each, 3.0e-16
+with base-2 ones, rounded twice; the test's line is a fifth above the first.
 """
 import numpy as np
 import pytest
@@ -149,3 +154,58 @@ def test_values_that_are_not_finite(engine):
             for i in range(len(x)):
                 close(out[i], exact(p[i])[0] + np.log(600 / 599), 2e-11)
         engine.lmode_free(tid)
+
+
+def test_rounding(engine):
+    ratio = []
+    for seed in range(30):
+        rng = np.random.default_rng(seed)
+        tab = sim.lmode_table(rng, 3000) * np.float32(2.0 ** rng.uniform(-1.5, 1.5))
+        x = np.column_stack([rng.uniform(0.5, 15, (30, 3)), rng.uniform(0.05, 4.0, (30, 2))])
+        tid = engine.lmode_table(np.ascontiguousarray(tab), 3, 2, 2)
+        out, _ = engine.jointp(tid, x, mode=L.LMODE_REF_COMPAT)
+        engine.lmode_free(tid)
+        t, v = tab.astype(np.longdouble), x.astype(np.longdouble)
+        err, size = [], []
+        cc, fc, hc, mc, fm = t[:, :3], t[:, 3:6], t[:, 6:9], t[:, 9:11], t[:, 11:13]
+        for i in range(len(x)):
+            p = (-t[:, 19] + cc @ (np.log(np.longdouble(2)) - np.log(v[i, :3])) - hc.sum(1)
+                 - (2 * fc) @ (1 / v[i, :3]) + mc @ np.log(v[i, 3:]) - fm @ v[i, 3:])
+            p = p[p > p.max() - 10]  # no list cap: values outside the window are kept first
+            want = np.log(np.longdouble(3000)) - (p.max() + np.log(np.exp(p - p.max()).sum()))
+            err.append(float(out[i] - want))
+            size.append(float(want))
+        ratio.append(np.linalg.norm(err) / np.linalg.norm(size))
+    assert np.sqrt(np.mean(np.square(ratio))) <= 1.2 * 2.2e-16
+
+
+def test_large_terms(engine):
+    """Base terms beyond 1e22 take the careful path, with padding behind them;
+    a term of -1.5e308 is still one."""
+    rng = np.random.default_rng(2)
+    for G in (1, 70, 300, 600, 40000):
+        tab = sim.lmode_table(rng, G)
+        x = points(rng, 20, 3, 2)
+        tab[:, 19] = 1e30
+        tid = engine.lmode_table(tab, 3, 2, 2)
+        out, _ = engine.jointp(tid, x, mode=L.LMODE_EXACT)
+        np.testing.assert_allclose(out, np.float64(np.float32(1e30)), rtol=1e-15)
+        engine.lmode_free(tid)
+    tab = np.zeros((1, 10), np.float32)
+    tab[0, 1] = 1e38  # fc
+    tid = engine.lmode_table(tab, 1, 1, 2)
+    fc = np.float64(tab[0, 1])
+    out, _ = engine.jointp(tid, np.array([[fc / 0.75e308, 1.0]]), mode=L.LMODE_EXACT)
+    np.testing.assert_allclose(out, 1.5e308, rtol=1e-15)
+    engine.lmode_free(tid)
+
+
+@pytest.mark.parametrize("row", [3, 300, 99999])
+def test_infinite_term_in_any_stage(engine, row):
+    """Two stages a chunk: a term of +inf gives no number wherever it stands."""
+    tab = sim.lmode_table(np.random.default_rng(3), 100000)
+    tab[row, 19] = -np.inf
+    tid = engine.lmode_table(tab, 3, 2, 2)
+    out, _ = engine.jointp(tid, points(np.random.default_rng(4), 70, 3, 2), mode=L.LMODE_EXACT)
+    assert np.isnan(out).all()
+    engine.lmode_free(tid)
