@@ -787,12 +787,17 @@ size_t jointp_work_bytes(const LTable &t, int npoints) {
   return (size_t)npoints * nc * 48 + 64;
 }
 
+// Dynamic LDS of a kernel with T tiles: rows and points, later the partials
+// (part bytes each) over them.  With the kernel's own (stat bytes) it stays
+// within the 64 KiB that every launch keeps to.
 template <int NR, int T>
-static void x_grid(const LArgs &a, dim3 *grid, size_t *lds) {
+constexpr size_t x_lds(size_t part) {
   using X = XShape<NR>;
-  *grid = dim3((a.npoints + 16 * T - 1) / (16 * T), a.nchunks);
-  *lds = std::max((size_t)(X::kLds + T * 16 * X::kKP) * 8,
-                  (size_t)16 * T * 16 * std::max(sizeof(XPart), sizeof(RefPart)));
+  return std::max((size_t)(X::kLds + T * 16 * X::kKP) * 8, (size_t)16 * T * 16 * part);
+}
+template <int NR, int T>
+constexpr bool x_fits(size_t part, size_t stat) {
+  return x_lds<NR, T>(part) + stat <= 65536;
 }
 
 // T tiles of points per workgroup, TS in the window sums (more registers a
@@ -800,22 +805,24 @@ static void x_grid(const LArgs &a, dim3 *grid, size_t *lds) {
 template <int NR, int T, int TS>
 static void launch_tiles(const LArgs &a, int mode, double *work, double *out, double *ess,
                          hipStream_t st) {
+  static_assert(x_fits<NR, T>(sizeof(XPart), T * 16 * 4), "jointp_exact's LDS");
+  static_assert(x_fits<NR, T>(sizeof(double), T * 16 * 4), "jointp_ref_max's LDS");
+  static_assert(x_fits<NR, TS>(sizeof(RefPart), TS * 16 * 4 + 20 * 16 * 8), "jointp_ref_sum's LDS");
   const dim3 per_point((a.npoints + 3) / 4);
-  dim3 grid;
-  size_t lds;
-  x_grid<NR, T>(a, &grid, &lds);
+  auto grid = [&](int tiles) { return dim3((a.npoints + 16 * tiles - 1) / (16 * tiles), a.nchunks); };
   if (mode == IMA_LMODE_EXACT) {
     XPart *part = reinterpret_cast<XPart *>(work);
-    hipLaunchKernelGGL((jointp_exact<NR, T>), grid, dim3(kXLanes), lds, st, a, part);
+    hipLaunchKernelGGL((jointp_exact<NR, T>), grid(T), dim3(kXLanes),
+                       (x_lds<NR, T>(sizeof(XPart))), st, a, part);
     hipLaunchKernelGGL(jointp_exact_final, per_point, dim3(256), 0, st, a, part, out, ess);
   } else {
     double *cmax = work, *mfin = cmax + (size_t)a.npoints * a.nchunks;
     RefPart *part = reinterpret_cast<RefPart *>(mfin + a.npoints);
-    hipLaunchKernelGGL((jointp_ref_max<NR, T>), grid, dim3(kXLanes), lds, st, a, cmax);
+    hipLaunchKernelGGL((jointp_ref_max<NR, T>), grid(T), dim3(kXLanes),
+                       (x_lds<NR, T>(sizeof(double))), st, a, cmax);
     hipLaunchKernelGGL(jointp_ref_prefix, per_point, dim3(256), 0, st, a, cmax, mfin);
-    x_grid<NR, TS>(a, &grid, &lds);
-    hipLaunchKernelGGL((jointp_ref_sum<NR, TS>), grid, dim3(kXLanes), lds, st, a, cmax, mfin,
-                       part);
+    hipLaunchKernelGGL((jointp_ref_sum<NR, TS>), grid(TS), dim3(kXLanes),
+                       (x_lds<NR, TS>(sizeof(RefPart))), st, a, cmax, mfin, part);
     hipLaunchKernelGGL(jointp_ref_final, per_point, dim3(256), 0, st, a, mfin, part, out, ess);
   }
 }
