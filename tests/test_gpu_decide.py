@@ -28,11 +28,15 @@ pytestmark = pytest.mark.gpu
 KINDS = ["hky", "is", "hky", "is", "sw", "hky"]
 
 
-def _setup(seed, C=8, prior=True):
+def _setup(seed, C=8, prior=True, pops=2):
     rng = np.random.default_rng(seed)
-    pt, theta, ts, mig = sim.im_model_two_pop(t=0.8, m12=0.4, m21=0.6)
+    pt, theta, ts, mig = (sim.im_model_two_pop(t=0.8, m12=0.4, m21=0.6) if pops == 2 else
+                          sim.im_model_random(rng, pops))
     model = immodel.build(pt, qmax=15.0, mmax=4.0)
-    samp = [4, 5]
+    samp = [4, 5] if pops == 2 else [2] * pops
+    if pops > 2:  # a migration rate of its own in every period
+        model.mig_wp = [[w] for wp in model.mig_wp for w in wp]
+        model.mmax = np.full(len(model.mig_wp), 4.0)
     e = Engine(0)
     mid = e.model_add(model) if prior else None
     loci, lids, base, As, u = [], [], [], [], []
@@ -79,7 +83,7 @@ def _setup(seed, C=8, prior=True):
     e.mc3_setup(C, Lc, first, np.tile(u, C), np.tile(kappa, C), betas, seed=seed,
                 precision=L.PREC_FP64, scale_width=0.3)
     if prior:
-        e.mc3_set_prior(np.tile(ts, (C, 1)), 5.0, 2)
+        e.mc3_set_prior(np.tile(ts, (C, 1)), 5.0, pops)
     return dict(e=e, rng=rng, model=model, samp=samp, loci=loci, As=As, u=np.array(u),
                 kappa=kappa, first=first, prop=prop, cur=cur, ts=np.asarray(ts, float),
                 sumlogk=sl, betas=betas, pt=pt, theta=theta, mig=mig, C=C, Lc=Lc)
@@ -181,6 +185,36 @@ def test_decisions_equal_the_oracle_bit_for_bit():
                if S["cur"][c][l] is not None and KINDS[l] == "hky")
     assert topo > 0
     # device sweeps continue from the accepted topologies
+    e.mc3_run(12, L.MC3_GRAPH | L.MC3_SCALE | L.MC3_RY1)
+    _check_state(S, tol=1e-9)
+    e.close()
+
+
+def test_decisions_of_more_than_64_parameters_equal_the_oracle():
+    """Six populations, 11 sizes and 70 rates: more parameters than lanes."""
+    S = _setup(404, C=6, pops=6)
+    e, C, Lc = S["e"], S["C"], S["Lc"]
+    assert S["model"].npsize + S["model"].nmig == 81
+    taken = 0
+    for _ in range(2):
+        props = _proposals(S)
+        _write(S, props)
+        h = S["rng"].normal(0.0, 30.0, C * Lc)
+        U = S["rng"].uniform(0.0, 1.0, C * Lc)
+        dec = e.mc3_decide(S["prop"], h, U)
+        for c in range(C):
+            g, pr = S["cur"][c], props[c * Lc:(c + 1) * Lc]
+            old, new = ([_loglik(S, l, x[l]) for l in range(Lc)] for x in (g, pr))
+            w, nw = ([oracle.treeweight(x[l], S["model"], S["ts"], S["samp"]) for l in range(Lc)]
+                     for x in (g, pr))
+            ref, *_ = oracle.updategenealogy_decisions(
+                [x[0] for x in old], w, [x[0] for x in new], nw, [x[1] for x in new],
+                h[c * Lc:(c + 1) * Lc], U[c * Lc:(c + 1) * Lc], S["betas"][c], S["model"])
+            assert list(dec[c].astype(bool)) == ref, (c, dec[c], ref)
+            S["cur"][c] = [pr[l] if ref[l] else g[l] for l in range(Lc)]
+        taken += int(dec.sum())
+        _check_state(S)
+    assert 0 < taken < 2 * C * Lc
     e.mc3_run(12, L.MC3_GRAPH | L.MC3_SCALE | L.MC3_RY1)
     _check_state(S, tol=1e-9)
     e.close()
