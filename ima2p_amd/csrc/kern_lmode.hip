@@ -902,6 +902,30 @@ __device__ inline double lanes_sum(double s) {
   return s;
 }
 
+// lanes_sum of T sums, the one of s[lane T / 64] in each lane.  The lanes of a
+// pair split the sums between them as long as there are several: 10 exchanges
+// for eight sums instead of 48, the same additions.
+template <int T, int H>
+__device__ __forceinline__ void split_sums(double (&s)[T], int lane) {
+  if constexpr (H > 0) {
+    constexpr int off = kWave * H / T;
+    const bool up = (lane & off) != 0;
+#pragma unroll
+    for (int t = 0; t < H; ++t) {
+      const double keep = up ? s[t + H] : s[t], give = up ? s[t] : s[t + H];
+      s[t] = keep + __shfl_xor(give, off, kWave);
+    }
+    split_sums<T, H / 2>(s, lane);
+  }
+}
+template <int T>
+__device__ __forceinline__ double lanes_sums(double (&s)[T], int lane) {
+  split_sums<T, T / 2>(s, lane);
+#pragma unroll
+  for (int off = kWave / T / 2; off > 0; off >>= 1) s[0] += __shfl_xor(s[0], off, kWave);
+  return s[0];
+}
+
 struct MArgs {
   const float *rows;
   int G, K, npsize, nmig, param, expo;
@@ -910,12 +934,13 @@ struct MArgs {
   int nx, nchunks, chunk_rows;
 };
 
-template <int T>
+template <int T, int Q>
 __global__ __launch_bounds__(kRowLanes) void margin_partial(MArgs a, double *work) {
-  __shared__ double sx[T], slx[T], part[kRowLanes / kWave][T];
-  const int p0 = blockIdx.x * T, np = min(T, a.nx - p0);
+  constexpr int N = T * Q;  // a workgroup's points, T at a time
+  __shared__ double sx[N], slx[N], part[kRowLanes / kWave][N];
+  const int p0 = blockIdx.x * N, np = min(N, a.nx - p0);
   const int chunk = blockIdx.y, tid = threadIdx.x;
-  if (tid < T) {
+  if (tid < N) {
     sx[tid] = a.x[p0 + min(tid, np - 1)];
     slx[tid] = log(sx[tid]);
   }
@@ -924,39 +949,35 @@ __global__ __launch_bounds__(kRowLanes) void margin_partial(MArgs a, double *wor
   const bool size = a.param < a.npsize;
   const int p = size ? a.param : a.param - a.npsize;
   const double lmean = log(a.meani);
-  double s[T] = {};
   const int gend = min(a.G, (chunk + 1) * a.chunk_rows);
-  for (int r = chunk * a.chunk_rows + tid; r < gend; r += kRowLanes) {
-    const float *g = a.rows + (size_t)r * a.K;
-    const float c = g[(size ? L.ccp : L.mcp) + p];
-    const double cnt = (double)(c >= 0 ? (long)(c + 0.5) : (long)(c - 0.5));  // INTEGERROUND
-    // (fused where written so, whatever T)
-    const double w = g[(size ? L.fcp : L.fmp) + p], q = g[(size ? L.qip : L.mip) + p];
-    if (size) {
-      const double h = g[L.hccp + p], w2 = 2 * w;
+#pragma unroll 1
+  for (int q0 = 0; q0 < np; q0 += T) {
+    double s[T] = {};
+    for (int r = chunk * a.chunk_rows + tid; r < gend; r += kRowLanes) {
+      const float *g = a.rows + (size_t)r * a.K;
+      const float c = g[(size ? L.ccp : L.mcp) + p];
+      const double cnt = (double)(c >= 0 ? (long)(c + 0.5) : (long)(c - 0.5));  // INTEGERROUND
+      // (fused where written so, whatever T; the last points' neighbours are
+      // copies of them)
+      const double w = g[(size ? L.fcp : L.fmp) + p], q = g[(size ? L.qip : L.mip) + p];
+      if (size) {
+        const double h = g[L.hccp + p], w2 = 2 * w;
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        if (t >= np) break;
-        s[t] += exp(fma(cnt, kLn2 - slx[t], -q) - h - w2 / sx[t]);
-      }
-    } else if (a.expo) {
+        for (int t = 0; t < T; ++t)
+          s[t] += exp(fma(cnt, kLn2 - slx[q0 + t], -q) - h - w2 / sx[q0 + t]);
+      } else if (a.expo) {
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        if (t >= np) break;
-        s[t] += exp(fma(-w, sx[t], fma(cnt, slx[t], fma(-sx[t], a.meani, -q + lmean))));
-      }
-    } else {
+        for (int t = 0; t < T; ++t)
+          s[t] += exp(fma(-w, sx[q0 + t],
+                          fma(cnt, slx[q0 + t], fma(-sx[q0 + t], a.meani, -q + lmean))));
+      } else {
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        if (t >= np) break;
-        s[t] += exp(fma(-w, sx[t], fma(cnt, slx[t], -q)));
+        for (int t = 0; t < T; ++t)
+          s[t] += exp(fma(-w, sx[q0 + t], fma(cnt, slx[q0 + t], -q)));
       }
     }
-  }
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const double v = lanes_sum(s[t]);
-    if (tid % kWave == 0) part[tid / kWave][t] = v;
+    const double sum = lanes_sums(s, tid % kWave);
+    if (tid % (kWave / T) == 0) part[tid / kWave][q0 + tid % kWave / (kWave / T)] = sum;
   }
   __syncthreads();
   if (tid >= np) return;
@@ -993,14 +1014,22 @@ hipError_t launch_margincalc(const LTable &t, int param, const double *x, int nx
   MArgs a{t.rows, t.G, t.K, t.npsize, t.nmig, param, expo,
           expo ? 1.0 / prior_mean : 1.0, x, nx, 0, 0};
   row_chunks(t.G, &a.nchunks, &a.chunk_rows);
-  // A workgroup takes 16 points where that leaves several workgroups a CU,
-  // else 2.
-  if ((int64_t)nx * a.nchunks >= 16 * 1024)
-    hipLaunchKernelGGL(margin_partial<16>, dim3((nx + 15) / 16, a.nchunks), dim3(kRowLanes), 0, st,
-                       a, work);
+  // A workgroup takes 8 points where that leaves 8 workgroups a CU, else 2 (64
+  // points on 1e6 rows: 179 us with 2).  It takes 32, 8 at a time, where a lane
+  // has no more than two rows, whose loads and sums of lanes these share, and 4
+  // workgroups a CU are left: 20000 points on 30000 rows 1.01 ms, with 8 a
+  // workgroup 1.30 (with 16 in a loop the compiler did not unroll, 1.40); but
+  // 350 points on 1e6 rows 539 us, with 8 485.
+  const int64_t pairs = (int64_t)nx * a.nchunks;
+  if (pairs >= 32 * 1024 && a.chunk_rows <= 2 * kRowLanes)
+    hipLaunchKernelGGL((margin_partial<8, 4>), dim3((nx + 31) / 32, a.nchunks), dim3(kRowLanes), 0,
+                       st, a, work);
+  else if (pairs >= 8 * 2048)
+    hipLaunchKernelGGL((margin_partial<8, 1>), dim3((nx + 7) / 8, a.nchunks), dim3(kRowLanes), 0,
+                       st, a, work);
   else
-    hipLaunchKernelGGL(margin_partial<2>, dim3((nx + 1) / 2, a.nchunks), dim3(kRowLanes), 0, st, a,
-                       work);
+    hipLaunchKernelGGL((margin_partial<2, 1>), dim3((nx + 1) / 2, a.nchunks), dim3(kRowLanes), 0,
+                       st, a, work);
   hipLaunchKernelGGL(margin_final, dim3((nx + 3) / 4), dim3(256), 0, st, a, logi, yadjust, work,
                      out);
   return hipGetLastError();

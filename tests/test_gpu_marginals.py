@@ -45,7 +45,8 @@ def _margin(tab, p, x, expo, mean):
 
 
 @pytest.mark.parametrize("G,nx", [(1, 3), (255, 1), (256, 16), (257, 17), (700, 500), (5000, 2),
-                                  (66000, 125), (66000, 131)])
+                                  (66000, 125), (66000, 131), (20000, 414), (20000, 415),
+                                  (66000, 260), (140000, 130)])
 def test_margincalc(engine, G, nx):
     rng = np.random.default_rng(G + nx)
     tab = _table(rng, G)
