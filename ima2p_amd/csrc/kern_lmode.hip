@@ -415,36 +415,43 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_exact(LArgs a, XPart *work)
   }
 }
 
-__device__ inline double wave_max(double v) {
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, kWave));
+// over the W lanes of a point
+template <int W>
+__device__ inline double group_max(double v) {
+  for (int off = W / 2; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, W));
   return v;
 }
-__device__ inline double wave_add(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+template <int W>
+__device__ inline double group_add(double v) {
+  for (int off = W / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, W);
   return v;
 }
 
-// One wavefront per point: lanes take the chunks in turn, then a butterfly
-// (a thread per point walking its chunks took 63 us for one point on 1e5
-// genealogies and 160 us for 4096 on 1e6).
+// W lanes per point take the chunks in turn, then a butterfly (a thread per
+// point walking its chunks took 63 us for one point on 1e5 genealogies and
+// 160 us for 4096 on 1e6).  A wavefront, or four lanes on the few chunks of a
+// small table (20000 points on 30 genealogies in REF_COMPAT: 202 us a call and
+// 167).  How many depends on the table alone, as the sums' order does.
+constexpr int kFewChunks = 16;
+template <int W>
 __global__ __launch_bounds__(256) void jointp_exact_final(LArgs a, const XPart *work, double *out,
                                                           double *ess) {
-  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
+  const int pt = blockIdx.x * (256 / W) + threadIdx.x / W;
+  const int lane = threadIdx.x % W;
   if (pt >= a.npoints) return;
   const XPart *w = work + (size_t)pt * a.nchunks;
   double M = -DBL_MAX;
-  for (int c = lane; c < a.nchunks; c += kWave) M = fmax(M, w[c].M);
-  M = wave_max(M);
+  for (int c = lane; c < a.nchunks; c += W) M = fmax(M, w[c].M);
+  M = group_max<W>(M);
   double s = 0.0, s2 = 0.0;
-  for (int c = lane; c < a.nchunks; c += kWave) {
+  for (int c = lane; c < a.nchunks; c += W) {
     if (w[c].s == 0.0) continue;
     const double sc = exp_any(w[c].M - M);
     s += w[c].s * sc;
     s2 += w[c].s2 * sc * sc;
   }
-  s = wave_add(s);
-  s2 = wave_add(s2);
+  s = group_add<W>(s);
+  s2 = group_add<W>(s2);
   if (lane == 0) {
     out[pt] = log((double)a.G) - (M + log(s));
     if (ess) ess[pt] = s * s / s2;
@@ -561,30 +568,31 @@ __device__ inline double one_term(const LArgs &a, const float *g, const double *
 }
 
 // Per point, cmax[c] becomes the maximum over the chunks before c, and mfin
-// the maximum over all: one wavefront per point, 64 chunks at a time.  A
+// the maximum over all: W lanes per point, W chunks at a time.  A
 // point whose first value (always kept) lies outside the final window needs
 // no further search for one: its cmax[c] are the final maximum.
+template <int W>
 __global__ __launch_bounds__(256) void jointp_ref_prefix(LArgs a, double *cmax, double *mfin) {
-  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
+  const int pt = blockIdx.x * (256 / W) + threadIdx.x / W;
+  const int lane = threadIdx.x % W;
   if (pt >= a.npoints) return;
   double *cm = cmax + (size_t)pt * a.nchunks;
   const double first = one_term(a, a.rows, a.x + (size_t)pt * (a.npsize + a.nmig));
   double before = -DBL_MAX;
-  for (int c0 = 0; c0 < a.nchunks; c0 += kWave) {
+  for (int c0 = 0; c0 < a.nchunks; c0 += W) {
     const int c = c0 + lane;
     double v = c < a.nchunks ? cm[c] : -DBL_MAX;
-    for (int off = 1; off < kWave; off <<= 1) {
-      const double o = __shfl_up(v, off, kWave);
+    for (int off = 1; off < W; off <<= 1) {
+      const double o = __shfl_up(v, off, W);
       if (lane >= off) v = fmax(v, o);
     }
-    const double up = __shfl_up(v, 1, kWave);
+    const double up = __shfl_up(v, 1, W);
     if (c < a.nchunks) cm[c] = lane ? fmax(before, up) : before;
-    before = fmax(before, __shfl(v, kWave - 1, kWave));
+    before = fmax(before, __shfl(v, W - 1, W));
   }
   if (lane == 0) mfin[pt] = before;
   if (before - first >= kWindow + 1.0)  // clear of rounding: the kernel takes its own first value
-    for (int c = lane; c < a.nchunks; c += kWave) cm[c] = before;
+    for (int c = lane; c < a.nchunks; c += W) cm[c] = before;
 }
 
 template <int NR, int T>
@@ -727,30 +735,31 @@ __global__ __launch_bounds__(kXLanes, 2) void jointp_ref_sum(LArgs a, const doub
   }
 }
 
-// One wavefront per point.
+// W lanes per point.
+template <int W>
 __global__ __launch_bounds__(256) void jointp_ref_final(LArgs a, const double *mfin,
                                                         const RefPart *part, double *out,
                                                         double *ess) {
-  const int pt = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
+  const int pt = blockIdx.x * (256 / W) + threadIdx.x / W;
+  const int lane = threadIdx.x % W;
   if (pt >= a.npoints) return;
   const RefPart *P = part + (size_t)pt * a.nchunks;
   const int maxz = ref_maxz(mfin[pt]);
   double sum = 0.0, sum2 = 0.0, minp = DBL_MAX;
   int cnt = 0, outside = 0;
-  for (int c = lane; c < a.nchunks; c += kWave) {
+  for (int c = lane; c < a.nchunks; c += W) {
     sum += P[c].sum;
     sum2 += P[c].sum2;
     minp = fmin(minp, P[c].minp);
     cnt += P[c].cnt;
     outside |= P[c].outside;
   }
-  sum = wave_add(sum);
-  sum2 = wave_add(sum2);
-  minp = -wave_max(-minp);
-  for (int off = 32; off > 0; off >>= 1) {
-    cnt += __shfl_xor(cnt, off, kWave);
-    outside |= __shfl_xor(outside, off, kWave);
+  sum = group_add<W>(sum);
+  sum2 = group_add<W>(sum2);
+  minp = -group_max<W>(-minp);
+  for (int off = W / 2; off > 0; off >>= 1) {
+    cnt += __shfl_xor(cnt, off, W);
+    outside |= __shfl_xor(outside, off, W);
   }
   if (lane != 0) return;
   if (!outside && cnt > 1) {  // the list cap drops the smallest kept value
@@ -808,22 +817,26 @@ static void launch_tiles(const LArgs &a, int mode, double *work, double *out, do
   static_assert(x_fits<NR, T>(sizeof(XPart), T * 16 * 4), "jointp_exact's LDS");
   static_assert(x_fits<NR, T>(sizeof(double), T * 16 * 4), "jointp_ref_max's LDS");
   static_assert(x_fits<NR, TS>(sizeof(RefPart), TS * 16 * 4 + 20 * 16 * 8), "jointp_ref_sum's LDS");
-  const dim3 per_point((a.npoints + 3) / 4);
+  const bool few = a.nchunks <= kFewChunks;
+  const dim3 per_point(few ? (a.npoints + 63) / 64 : (a.npoints + 3) / 4);
   auto grid = [&](int tiles) { return dim3((a.npoints + 16 * tiles - 1) / (16 * tiles), a.nchunks); };
   if (mode == IMA_LMODE_EXACT) {
     XPart *part = reinterpret_cast<XPart *>(work);
     hipLaunchKernelGGL((jointp_exact<NR, T>), grid(T), dim3(kXLanes),
                        (x_lds<NR, T>(sizeof(XPart))), st, a, part);
-    hipLaunchKernelGGL(jointp_exact_final, per_point, dim3(256), 0, st, a, part, out, ess);
+    hipLaunchKernelGGL(few ? jointp_exact_final<4> : jointp_exact_final<kWave>, per_point,
+                       dim3(256), 0, st, a, part, out, ess);
   } else {
     double *cmax = work, *mfin = cmax + (size_t)a.npoints * a.nchunks;
     RefPart *part = reinterpret_cast<RefPart *>(mfin + a.npoints);
     hipLaunchKernelGGL((jointp_ref_max<NR, T>), grid(T), dim3(kXLanes),
                        (x_lds<NR, T>(sizeof(double))), st, a, cmax);
-    hipLaunchKernelGGL(jointp_ref_prefix, per_point, dim3(256), 0, st, a, cmax, mfin);
+    hipLaunchKernelGGL(few ? jointp_ref_prefix<4> : jointp_ref_prefix<kWave>, per_point,
+                       dim3(256), 0, st, a, cmax, mfin);
     hipLaunchKernelGGL((jointp_ref_sum<NR, TS>), grid(TS), dim3(kXLanes),
                        (x_lds<NR, TS>(sizeof(RefPart))), st, a, cmax, mfin, part);
-    hipLaunchKernelGGL(jointp_ref_final, per_point, dim3(256), 0, st, a, mfin, part, out, ess);
+    hipLaunchKernelGGL(few ? jointp_ref_final<4> : jointp_ref_final<kWave>, per_point,
+                       dim3(256), 0, st, a, mfin, part, out, ess);
   }
 }
 
