@@ -246,7 +246,6 @@ hipError_t launch_margincalc(const LTable &t, int param, const double *x,
                              double prior_mean, double *work, double *out,
                              hipStream_t st);
 size_t margincalc_work_bytes(const LTable &t, int nx);
-hipError_t upload_pow10_table(hipStream_t st);
 
 // Genealogy prior (kern_prior.hip).
 size_t treeweight_lds_bytes(int P, int emax);   // the bound on a genealogy's events

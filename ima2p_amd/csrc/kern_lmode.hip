@@ -12,7 +12,9 @@
 // Chunk partials are merged by a second kernel in a fixed order, and the
 // rows a lane works on depend on the table only, never on how many points
 // share a launch, so a point's result is the same alone and batched with
-// others.  margincalc: one thread per value, 64-value tiles.
+// others.  margincalc and the 2NM density have rows on the lanes, the 2NM
+// density of many points has points; a point's value is the same in any batch
+// there too.
 #include <float.h>
 #include <limits.h>
 
@@ -22,8 +24,6 @@
 #include "prior_math.h"
 
 namespace ima {
-
-constexpr int kLStage = 128;    // rows staged in LDS at a time
 
 struct JointLayout {
   int ccp, fcp, hccp, mcp, fmp, qip, mip, pdgp, probgp;
@@ -771,19 +771,15 @@ __global__ __launch_bounds__(256) void jointp_ref_final(LArgs a, const double *m
   if (ess) ess[pt] = sum * sum / sum2;
 }
 
-// Rows staged in LDS at a time (FP64 rows, at most 32 KB) and rows per
-// chunk: a function of the table alone, aiming at about 256 chunks.
-static int stage_of(const LTable &t) {
-  int st = 32768 / (8 * t.K);
-  st = st >= kLStage ? kLStage : (st / 8) * 8;
-  return st < 8 ? 8 : st;
-}
-static void chunking(const LTable &t, int npoints, int *nchunks, int *chunk_rows) {
-  (void)npoints;
-  const int st = stage_of(t);
+// jointp's rows per chunk, a function of the table alone: about 256 chunks, in
+// steps of 128 rows (fewer where 128 rows of FP64 exceed 32 KB).  The work
+// area's size, and with it the calls that are refused, follows from these; the
+// kernels round them up to whole stages (launch_nr), so they make no more
+// chunks than it has room for.
+static void chunking(const LTable &t, int *nchunks, int *chunk_rows) {
+  const int step = std::max(8, std::min(128, 32768 / (8 * t.K) / 8 * 8));
   int rows = (t.G + 255) / 256;
-  rows = ((rows + st - 1) / st) * st;
-  if (rows < st) rows = st;
+  rows = std::max(step, (rows + step - 1) / step * step);
   *chunk_rows = rows;
   *nchunks = (t.G + rows - 1) / rows;
 }
@@ -792,7 +788,7 @@ static void chunking(const LTable &t, int npoints, int *nchunks, int *chunk_rows
 // many chunks as `chunking` makes (the kernels' own chunks are no smaller).
 size_t jointp_work_bytes(const LTable &t, int npoints) {
   int nc, cr;
-  chunking(t, npoints, &nc, &cr);
+  chunking(t, &nc, &cr);
   return (size_t)npoints * nc * 48 + 64;
 }
 
@@ -870,7 +866,7 @@ hipError_t launch_jointp(const LTable &t, const double *x, int npoints, int mode
                          double *out, double *ess, hipStream_t st) {
   if (npoints == 0) return hipSuccess;
   LArgs a{t.rows, t.G, t.K, t.npsize, t.nmig, t.npops, modeltype, r0, r1, x, npoints, 0, 0};
-  chunking(t, npoints, &a.nchunks, &a.chunk_rows);
+  chunking(t, &a.nchunks, &a.chunk_rows);
   if (jointp_work_bytes(t, npoints) > work_bytes) return hipErrorInvalidValue;
   switch (r1 - r0) {
 #define IMA_NR(N) \
@@ -1596,7 +1592,5 @@ hipError_t launch_greater_than(const LTable &t, int kind, const int2 *pairs, con
   hipLaunchKernelGGL(gt_mean, dim3(npairs), dim3(64), 0, st, a, per, out);
   return hipGetLastError();
 }
-
-hipError_t upload_pow10_table(hipStream_t) { return hipSuccess; }
 
 }  // namespace ima

@@ -483,7 +483,7 @@ __device__ inline bool param_hit(const ModelView &md, int P, int npsize, int t,
 // the records' first kRecRegs * 64 entries through registers.
 constexpr int kRecRegs = 3;
 struct LocusFetch {
-  double o[kRecRegs], n[kRecRegs], npd, pdg, lu;
+  double o[kRecRegs], n[kRecRegs], npd, pdg;
   int ok;
 };
 __device__ __forceinline__ void prior_load(const MC3Dev &m, int it, LocusFetch &f) {
