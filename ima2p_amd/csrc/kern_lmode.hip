@@ -1289,13 +1289,13 @@ __global__ __launch_bounds__(256) void popmig_final(PArgs a, const double *work,
 // what the chip holds (4096) and 64 points are not mostly padding; then 16
 // leaves a wavefront where those fill the chip, else four.  Calls in us (25
 // of them copies and waiting), uniform prior:
-//   20000 rows, 1 point:     42 with rows, 118 with points (16 leaves)
-//   20000 rows, 100 points:  160, 180
-//   20000 rows, 256 points:  330, 252 (four leaves: 286)
-//   20000 rows, 500 points:  593, 399
-//   2000 rows, 256 points:   77, 117 (84)
-//   2000 rows, 500 points:   104, 116 (86)
-//   2000 rows, 2000 points:  285, 204 (229)
+//   20000 rows, 1 point:     42 with rows, 122 with points (16 leaves)
+//   20000 rows, 100 points:  163, 182
+//   20000 rows, 256 points:  342, 258 (four leaves: 283)
+//   20000 rows, 500 points:  602, 409
+//   2000 rows, 256 points:   77, 118 (84)
+//   2000 rows, 500 points:   107, 119 (85)
+//   2000 rows, 2000 points:  290, 206 (228)
 PopmigPlan popmig_plan(int n, int nx, int expo) {
   PopmigPlan p;
   const int leaf = (n - 1) / (1024 * kWave) + 1;

@@ -265,8 +265,8 @@ constexpr double kDown95 = 1.92;    // DOWN95
 // values: the same points in the same order decide it, in 1/depth of the
 // launches.  depth grows while the extra terms stay cheap beside a launch
 // (terms: how many of the density's kind take 10 to 20 us).  The peaks and 95% limits of one parameter on
-// 20000 genealogies: 2.7 ms point by point, 0.45 ms with depth 6; a 2NM peak
-// 1.4 and 0.6 ms with depth 4.
+// 20000 genealogies: 2.7 ms point by point, 0.26 to 0.52 ms with depth 6; a 2NM
+// peak 1.4 and 0.6 ms with depth 4.
 int search_depth(int G, int64_t terms, int most) {
   int d = 1;
   while (d < most && (((int64_t)2 << d) - 1) * G <= terms) ++d;
