@@ -7,11 +7,11 @@ where a workgroup takes more points or the lanes change from rows to points.
   parts up to a few hundred, is within 4 roundings of each (1e-13), and the
   sum's order gives less: 1e-12.  A point's value must have the same bits in
   every batch.
-* popmig: both layouts sum the same positive terms: G * 2^-52, times 2 for the
-  exponential prior's changes of reference, and the rounding of a term's log
-  where the compiler fuses another product in the other kernel: parts up to
-  500, ten of them, 10 * 500 * 2^-53 = 6e-13.
-  A point's value must have the same bits in every batch all the same.
+* popmig: both layouts add the same tree of terms, so a point's value must have
+  the same bits in every batch.  The test of batches of 100 against larger
+  ones allows for the same positive terms in another order (G * 2^-52, twice
+  that for the exponential prior's changes of reference) with another rounding
+  of a term's log: parts up to 500, ten of them, 10 * 500 * 2^-53 = 6e-13.
 * peaks and limits must equal, bit for bit, the searches run here one point
   at a time; 2NM peaks with the same number of points."""
 import numpy as np

@@ -5,7 +5,7 @@ Integrals: counts from none to thousands, weights from far below to far
 above the priors' bounds (either end of the incomplete gammas: series,
 continued fraction, saturated), against the oracle.  Bound: both stop their
 series at the same term (relative 3e-7, the comparison rounds at 1e-16), and
-the logarithms of at most 1e5 in size that make an integral are within 2 ulp,
+the logarithms of at most 1e5 in size that make an integral are within an ulp,
 so the values agree to 1e-15 of the largest of them; the tolerance is the
 path's own 1e-10 relative, with 1e-9 absolute for values near zero.
 
